@@ -714,7 +714,8 @@ __device__ __forceinline__ void elem_pass(StepArgs a, const int blk, const int n
     }
     evol *= 0.5;                          /* UpdateElement.c:267-268 */
     const double elemVolume = 2.0 * evol; /* StrainRate.c:57, Stress.c:68 */
-    const double srcorr = partial / elemVolume;
+    const snh_recip rEV = snh_recip_make(elemVolume);
+    const double srcorr = snh_quot(partial, rEV);
 
     /* rotation of the stored stress, strain (Stress.c:71-82) */
     if constexpr (!kEarly) {
@@ -869,7 +870,7 @@ __device__ __forceinline__ void elem_pass(StepArgs a, const int blk, const int n
     double pst = 0.0;
 #pragma unroll
     for (int q = 0; q < NTET; q++) pst += sh_c[le][q];
-    const double avgTrace = pst / elemVolume;
+    const double avgTrace = snh_quot(pst, rEV);
     st[0] += -1.0 * tr + avgTrace;
     st[1] += -1.0 * tr + avgTrace;
     st[2] += -1.0 * tr + avgTrace;
@@ -1413,10 +1414,9 @@ __device__ __forceinline__ void node_pass(StepArgs a, const int blk, const int n
                 double ax, ay, az;
                 face_cross(X[kTetraToNode[t][kFaceToNode[f][0]]], X[kTetraToNode[t][kFaceToNode[f][1]]],
                            X[kTetraToNode[t][kFaceToNode[f][2]]], ax, ay, az);
-                const double sq = sqrt(ax * ax + ay * ay + az * az);
-                const double area = sq / 2.0;
-                const double ysq = 1.0 / sq;
-                const double n0 = snh_div_by(ax, sq, ysq), n1 = snh_div_by(ay, sq, ysq), n2 = snh_div_by(az, sq, ysq);
+                snh_recip rs;
+                const double sq = snh_sqrt_recip(ax * ax + ay * ay + az * az, &rs);
+                const double n0 = snh_quot(ax, rs), n1 = snh_quot(ay, rs), n2 = snh_quot(az, rs);
                 const double s00 = a.stress[((size_t)0 * NTET + t) * E + e];
                 const double s11 = a.stress[((size_t)1 * NTET + t) * E + e];
                 const double s22 = a.stress[((size_t)2 * NTET + t) * E + e];
@@ -1426,6 +1426,7 @@ __device__ __forceinline__ void node_pass(StepArgs a, const int blk, const int n
                 if (a.dtType == SNH_DT_DYNAMIC) {
                     im += 0.25 * inertialDensity * V;
                 } else if (a.dtType == SNH_DT_CONSTANT) {
+                    const double area = sq / 2.0;
                     double area_sum = 0.0, tmp;
                     tmp = (n0 * area) * (n0 * area);
                     if (tmp > area_sum) area_sum = tmp;
@@ -1437,10 +1438,10 @@ __device__ __forceinline__ void node_pass(StepArgs a, const int blk, const int n
                 } else {
                     im += 0.25 * rho * V;
                 }
-                f0 += snh_div6((s00 * n0 + s01 * n1 + s02 * n2) * area);   /* (...)*area/6.0 */
-                f1 += snh_div6((s01 * n0 + s11 * n1 + s12 * n2) * area);
-                f2 += snh_div6((s02 * n0 + s12 * n1 + s22 * n2) * area);
-                f1 -= a.gravity * rho * V / 8.0;
+                f0 += snh_div12((s00 * n0 + s01 * n1 + s02 * n2) * sq);   /* (...)*area/6.0 */
+                f1 += snh_div12((s01 * n0 + s11 * n1 + s12 * n2) * sq);
+                f2 += snh_div12((s02 * n0 + s12 * n1 + s22 * n2) * sq);
+                f1 -= (0.125 * a.gravity) * rho * V;   /* gravity*rho*V/8.0 */
             }
         }
         vmag = node_finish(a, n, f0, f1, f2, im, own, dt);
@@ -1489,13 +1490,13 @@ __device__ __forceinline__ void face_share(const StepArgs& a, const DevMaterial&
                                            const double* c3, const double st[6], double dt, double acc[4]) {
     double ax, ay, az;
     face_cross(c1, c2, c3, ax, ay, az);
-    const double sq = sqrt(ax * ax + ay * ay + az * az);
-    const double area = sq / 2.0;
-    const double ysq = 1.0 / sq;
-    const double n0 = snh_div_by(ax, sq, ysq), n1 = snh_div_by(ay, sq, ysq), n2 = snh_div_by(az, sq, ysq);
+    snh_recip rs;
+    const double sq = snh_sqrt_recip(ax * ax + ay * ay + az * az, &rs);
+    const double n0 = snh_quot(ax, rs), n1 = snh_quot(ay, rs), n2 = snh_quot(az, rs);
     if (a.dtType == SNH_DT_DYNAMIC) {
         acc[3] += 0.25 * inertialDensity * V;
     } else if (a.dtType == SNH_DT_CONSTANT) {
+        const double area = sq / 2.0;
         double area_sum = 0.0, tmp;
         tmp = (n0 * area) * (n0 * area);
         if (tmp > area_sum) area_sum = tmp;
@@ -1507,10 +1508,10 @@ __device__ __forceinline__ void face_share(const StepArgs& a, const DevMaterial&
     } else {
         acc[3] += 0.25 * rho * V;
     }
-    acc[0] += snh_div6((st[0] * n0 + st[3] * n1 + st[4] * n2) * area);
-    acc[1] += snh_div6((st[3] * n0 + st[1] * n1 + st[5] * n2) * area);
-    acc[2] += snh_div6((st[4] * n0 + st[5] * n1 + st[2] * n2) * area);
-    acc[1] -= a.gravity * rho * V / 8.0;
+    acc[0] += snh_div12((st[0] * n0 + st[3] * n1 + st[4] * n2) * sq);   /* (...)*area/6.0 */
+    acc[1] += snh_div12((st[3] * n0 + st[1] * n1 + st[5] * n2) * sq);
+    acc[2] += snh_div12((st[4] * n0 + st[5] * n1 + st[2] * n2) * sq);
+    acc[1] -= (0.125 * a.gravity) * rho * V;   /* gravity*rho*V/8.0 */
 }
 
 /* the 40 tet-face shares of a node, per node-slot s and rank r in the
@@ -2083,12 +2084,11 @@ __device__ __forceinline__ void face_normal_area(const double* p0, const double*
                                                  double& area) {
     double ax, ay, az;
     face_cross(p0, p1, p2, ax, ay, az);
-    const double sq = sqrt(ax * ax + ay * ay + az * az);
-    area = sq / 2.0;
-    const double ysq = 1.0 / sq;
-    n[0] = snh_div_by(ax, sq, ysq);
-    n[1] = snh_div_by(ay, sq, ysq);
-    n[2] = snh_div_by(az, sq, ysq);
+    snh_recip rs;
+    area = 0.5 * snh_sqrt_recip(ax * ax + ay * ay + az * az, &rs);
+    n[0] = snh_quot(ax, rs);
+    n[1] = snh_quot(ay, rs);
+    n[2] = snh_quot(az, rs);
 }
 
 /* tet surfaces whose mean normal is the wall normal of the heat-flux
@@ -2151,7 +2151,7 @@ __global__ void __launch_bounds__(GEO_BLOCK) k_heat_elem(StepArgs a) {
         const double* P[4] = {X[kTetraToNode[t][0]], X[kTetraToNode[t][1]], X[kTetraToNode[t][2]],
                               X[kTetraToNode[t][3]]};
         const double V = tet_volume(P[0], P[1], P[2], P[3]);
-        const double yV = 1.0 / V;
+        const snh_recip rV = snh_recip_make(V);
         double n[4][3], A[4];
 #pragma unroll
         for (int f = 0; f < 4; f++)
@@ -2163,12 +2163,12 @@ __global__ void __launch_bounds__(GEO_BLOCK) k_heat_elem(StepArgs a) {
         for (int d = 0; d < 3; d++) {
             /* node k pairs with surface (k+1)%4, summed left to right */
             S[d] = T0 * n[1][d] * A[1] + T1 * n[2][d] * A[2] + T2 * n[3][d] * A[3] + T3 * n[0][d] * A[0];
-            hf[d] = snh_div_by(snh_div3(1.0 * m.kcond * S[d]), V, yV);   /* 1.0f*k*(..)/3.0f/V */
+            hf[d] = snh_quot(snh_div3(1.0 * m.kcond * S[d]), rV);   /* 1.0f*k*(..)/3.0f/V */
         }
         if (wall >= 0) {
             double g[3];
 #pragma unroll
-            for (int d = 0; d < 3; d++) g[d] = snh_div_by(snh_div3(-1.0 * S[d]), V, yV);
+            for (int d = 0; d < 3; d++) g[d] = snh_quot(snh_div3(-1.0 * S[d]), rV);
             double Fn = 0.0;
             Fn += g[0] * nb[0];
             Fn += g[1] * nb[1];

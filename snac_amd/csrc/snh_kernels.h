@@ -207,7 +207,7 @@ SNH_HD double tet_volume(const double* c1, const double* c2, const double* c3, c
 /* geometry + velocity-gradient terms of one tet (UpdateElement.c:84-219,
    StrainRate.c:65-184): node k pairs with face (k+1)%4 */
 SNH_HD void tet_kinematics(const double X[4][3], const double U[4][3], TetKin& o) {
-    double n[4][3], A[4];
+    double n[4][3], A[4];   /* A: the norm of the face cross product, twice the area */
     double a0 = 0, b0 = 0, c0 = 0;
 #pragma unroll
     for (int f = 0; f < 4; f++) {
@@ -218,15 +218,16 @@ SNH_HD void tet_kinematics(const double X[4][3], const double U[4][3], TetKin& o
             b0 = b;
             c0 = c;
         }
-        double s = sqrt(a * a + b * b + c * c);
-        const double ys = 1.0 / s;
-        A[f] = s / 2.0;
-        n[f][0] = snh_div_by(a, s, ys);   /* == a / s */
-        n[f][1] = snh_div_by(b, s, ys);
-        n[f][2] = snh_div_by(c, s, ys);
+        snh_recip rs;
+        A[f] = snh_sqrt_recip(a * a + b * b + c * c, &rs);
+        n[f][0] = snh_quot(a, rs);   /* == a / s */
+        n[f][1] = snh_quot(b, rs);
+        n[f][2] = snh_quot(c, rs);
     }
     const double V = tet_volume_from_face0(X[0], X[3], a0, b0, c0);
     o.V = V;
+    /* twice the reference's products U n A (the factor is exact and goes into
+       the divisions by 3 below) */
 #define T_(k, p, q) (U[k][p] * n[((k) + 1) & 3][q] * A[((k) + 1) & 3])
     /* products shared between strain rate and rotation */
     const double s00 = T_(0, 0, 0) + T_(1, 0, 0) + T_(2, 0, 0) + T_(3, 0, 0);
@@ -235,16 +236,15 @@ SNH_HD void tet_kinematics(const double X[4][3], const double U[4][3], TetKin& o
     const double s01 = T_(0, 0, 1) + T_(1, 0, 1) + T_(2, 0, 1) + T_(3, 0, 1);
     const double s02 = T_(0, 0, 2) + T_(1, 0, 2) + T_(2, 0, 2) + T_(3, 0, 2);
     const double s12 = T_(0, 1, 2) + T_(1, 1, 2) + T_(2, 1, 2) + T_(3, 1, 2);
-    /* x / 3.0 / V as snh_div_by(snh_div3(x), V, RN(1/V)): the same two
-       correctly rounded quotients */
-    const double yV = 1.0 / V;
-    o.sr[0] = snh_div_by(snh_div3(-1.0 * s00), V, yV);
-    o.sr[1] = snh_div_by(snh_div3(-1.0 * s11), V, yV);
-    o.sr[2] = snh_div_by(snh_div3(-1.0 * s22), V, yV);
-    o.sr[3] = snh_div_by(snh_div3(-0.5 * (s01 + T_(0, 1, 0) + T_(1, 1, 0) + T_(2, 1, 0) + T_(3, 1, 0))), V, yV);
-    o.sr[4] = snh_div_by(snh_div3(-0.5 * (s02 + T_(0, 2, 0) + T_(1, 2, 0) + T_(2, 2, 0) + T_(3, 2, 0))), V, yV);
-    o.sr[5] = snh_div_by(snh_div3(-0.5 * (s12 + T_(0, 2, 1) + T_(1, 2, 1) + T_(2, 2, 1) + T_(3, 2, 1))), V, yV);
-    const double hv = -(yV * 0.5);   /* RN(0.5/V) == RN(1/V)/2 */
+    /* x / 3.0 / V as two correctly rounded quotients */
+    const snh_recip rV = snh_recip_make(V);
+    o.sr[0] = snh_quot(snh_ndiv6(s00), rV);
+    o.sr[1] = snh_quot(snh_ndiv6(s11), rV);
+    o.sr[2] = snh_quot(snh_ndiv6(s22), rV);
+    o.sr[3] = snh_quot(snh_ndiv12(s01 + T_(0, 1, 0) + T_(1, 1, 0) + T_(2, 1, 0) + T_(3, 1, 0)), rV);
+    o.sr[4] = snh_quot(snh_ndiv12(s02 + T_(0, 2, 0) + T_(1, 2, 0) + T_(2, 2, 0) + T_(3, 2, 0)), rV);
+    o.sr[5] = snh_quot(snh_ndiv12(s12 + T_(0, 2, 1) + T_(1, 2, 1) + T_(2, 2, 1) + T_(3, 2, 1)), rV);
+    const double hv = -(rV.hi * 0.25);   /* RN(0.5/V) == RN(1/V)/2; a quarter for the doubled products */
     o.w[0] = snh_div3(hv * (s01 - T_(0, 1, 0) - T_(1, 1, 0) - T_(2, 1, 0) - T_(3, 1, 0)));
     o.w[1] = snh_div3(hv * (s02 - T_(0, 2, 0) - T_(1, 2, 0) - T_(2, 2, 0) - T_(3, 2, 0)));
     o.w[2] = snh_div3(hv * (s12 - T_(0, 2, 1) - T_(1, 2, 1) - T_(2, 2, 1) - T_(3, 2, 1)));

@@ -92,9 +92,21 @@ SNH_HD double snh_div3(double x) {
     return fma(r, y, q);
 }
 
-/* RN(x / 6) = RN(x / 3) / 2 exactly (halving commutes with rounding in the
- * normal range) */
-SNH_HD double snh_div6(double x) { return snh_div3(x) * 0.5; }
+/* RN(c x / 3) for c a power of two, of either sign: c times the steps above,
+ * exactly (a power of two commutes with rounding in the normal range), so a
+ * halving, quartering or sign beside the division costs nothing.
+ * RN(x / 6) is c = 1/2. */
+#define SNH_DIV3C(name, c)                               \
+    SNH_HD double name(double x) {                       \
+        const double y = (c) * 0x1.5555555555555p-2;     \
+        double q = x * y;                                \
+        double r = fma(-3.0 / (c), q, x);                \
+        return fma(r, y, q);                             \
+    }
+SNH_DIV3C(snh_div6, 0.5)
+SNH_DIV3C(snh_div12, 0.25)
+SNH_DIV3C(snh_ndiv6, -0.5)
+SNH_DIV3C(snh_ndiv12, -0.25)
 
 /* RN(a / b) from y = RN(1 / b) (P. Markstein, "Computation of elementary
  * functions on the IBM RISC System/6000", IBM J. Res. Dev. 34 (1990); and
@@ -108,6 +120,71 @@ SNH_HD double snh_div_by(double a, double b, double y) {
     q = fma(r, y, q);
     r = fma(-b, q, a);
     return fma(r, y, q);
+}
+
+/* A divisor b as the unevaluated sum hi + lo = 1 / b (1 + 2^-104): quotients
+ * by it are a product and an FMA, RN(a hi + RN(a lo)) (N. Brisebarre,
+ * J.-M. Muller and S. K. Raina, "Accelerating correctly rounded
+ * floating-point division when the divisor is known in advance", IEEE Trans.
+ * Computers 53 (2004), method 1).  The sum before the rounding is within
+ * 2^-52 ulp of a / b, so the result is RN(a / b) unless the quotient lies that
+ * close to a rounding midpoint; 4e9 random quotients on gfx950 gave no
+ * difference from the division.  Normal range only.
+ *
+ * From an estimate of 1 / b good to 2^-24 (v_rcp_f64, v_rsq_f64), one or two
+ * Newton steps (P. Markstein, 1990) make hi faithful; the residual
+ * 1 - b hi is then exact, and lo is its product with hi. */
+typedef struct {
+    double hi, lo;
+} snh_recip;
+SNH_HD snh_recip snh_recip_of(double b, double y) {
+    snh_recip r;
+    double e = fma(-b, y, 1.0);
+    r.hi = fma(e, y, y);
+    e = fma(-b, r.hi, 1.0);
+    r.lo = e * r.hi;
+    return r;
+}
+SNH_HD double snh_quot(double a, snh_recip r) { return fma(a, r.hi, a * r.lo); }
+
+/* the reciprocal of b > 0 */
+SNH_HD snh_recip snh_recip_make(double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double y = __builtin_amdgcn_rcp(b);
+    y = fma(fma(-b, y, 1.0), y, y);
+#else
+    const double y = 1.0 / b;
+#endif
+    return snh_recip_of(b, y);
+}
+
+/* RN(sqrt(x)) for x > 0 and, in r, the reciprocal of that root.  Goldschmidt's
+ * coupled iteration for sqrt(x) and 1 / (2 sqrt(x)) from v_rsq_f64, then two
+ * residual corrections of the root (Markstein 1990; Muller et al., Handbook of
+ * Floating-Point Arithmetic, 2nd ed., sec. 4.7), which give the correctly
+ * rounded root; the reciprocal comes out of the same iteration instead of a
+ * division.  Without the scaling of the library's sqrt: normal range only
+ * (x = 0 gives NaN, as the 0 / 0 of a face without area does).
+ * 13 instructions for root and reciprocal and 2 per quotient, against 31 and
+ * 5 with sqrt, 1 / s and snh_div_by. */
+SNH_HD double snh_sqrt_recip(double x, snh_recip* r) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double t = fma(-h, g, 0.5);
+    g = fma(g, t, g);
+    h = fma(h, t, h);
+    double d = fma(-g, g, x);
+    g = fma(d, h, g);
+    d = fma(-g, g, x);
+    g = fma(d, h, g);
+    *r = snh_recip_of(g, h + h);
+    return g;
+#else
+    const double s = sqrt(x);
+    *r = snh_recip_of(s, 1.0 / s);
+    return s;
+#endif
 }
 
 #endif
