@@ -258,7 +258,7 @@ class Context:
         shapes = {"coord": (self.N, 3), "velocity": (self.N, 3), "stress": (self.E, 10, 6),
                   "plastic_strain": (self.E, 10), "viscosity": (self.E, 10), "volume": (self.E, 10),
                   "temperature": (self.N,)}
-        out = {f: np.zeros(shapes[f]) for f in fields}
+        out = {f: np.empty(shapes[f]) for f in fields}   # every one is filled
         st = _abi.State()
         for f, a in out.items():
             setattr(st, f, _dp(a))

@@ -35,6 +35,7 @@
 
 #include "../../include/snac_hip.h"
 #include "snh_kernels.h"
+#include "snh_landing.h"
 
 using namespace snh;
 
@@ -3401,6 +3402,7 @@ extern "C" int snh_context_create(const snh_config* cfg, snh_context** out) {
     c->zero_done = false;
     c->rotation_pending = false;
     c->timeStep = 0;
+    land_context_made();
     *out = c;
     return SNH_OK;
 }
@@ -3415,6 +3417,7 @@ extern "C" int snh_context_destroy(snh_context* c) {
     free_all(c);
     if (c->own_stream) (void)hipStreamDestroy(c->stream);
     delete c;
+    land_context_gone();
     return SNH_OK;
 }
 
@@ -3475,7 +3478,7 @@ static int ensure_stage(snh_context* c) {
 }
 
 /* device rows -> host records of one field */
-static int download_rows(snh_context* c, const double* rows, double* host, size_t M, int kind) {
+static int download_rows(snh_context* c, Landing& land, const double* rows, double* host, size_t M, int kind) {
     int rc;
     if ((rc = ensure_stage(c))) return rc;
     const dim3 grid((unsigned)((M + 63) / 64)), block(256);
@@ -3486,8 +3489,7 @@ static int download_rows(snh_context* c, const double* rows, double* host, size_
     default: C = 60; hipLaunchKernelGGL((k_rows_to_records<60, LAY_STRESS>), grid, block, 0, c->stream, rows, c->stage, M); break;
     }
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(host, c->stage, C * M * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(land.push(host, c->stage, C * M * sizeof(double)));
     return SNH_OK;
 }
 
@@ -4214,12 +4216,15 @@ extern "C" int snh_download_state(snh_context* c, snh_state* s) {
     if (!c || !s) return set_err(SNH_EINVAL, "null argument");
     const size_t N = c->N, E = c->E;
     int rc;
-    HIPCHK(hipStreamSynchronize(c->stream));
     if (s->temperature && !c->thermal)
         return set_err(SNH_EINVAL, "no temperature plugin in this context (snh_set_thermal)");
-    if (s->coord && (rc = download_rows(c, c->x[c->cur], s->coord, N, XF_VEC3))) return rc;
-    if (s->temperature) HIPCHK(ctx_copy(c, s->temperature, c->temp, N * sizeof(double), hipMemcpyDeviceToHost));
-    if (s->velocity && (rc = download_rows(c, c->v, s->velocity, N, XF_VEC3))) return rc;
+    const bool ps = s->plastic_strain && c->ps, visc = s->viscosity && c->visc;
+    Landing land(c->stream, sizeof(double) * (N * ((s->coord ? 3 : 0) + (s->velocity ? 3 : 0) + (s->temperature ? 1 : 0)) +
+                                              E * ((s->stress ? 60 : 0) + (s->volume ? 10 : 0) + (ps ? 10 : 0) +
+                                                   (visc ? 10 : 0))));
+    if (s->coord && (rc = download_rows(c, land, c->x[c->cur], s->coord, N, XF_VEC3))) return rc;
+    if (s->temperature) HIPCHK(land.push(s->temperature, c->temp, N * sizeof(double)));
+    if (s->velocity && (rc = download_rows(c, land, c->v, s->velocity, N, XF_VEC3))) return rc;
     if (s->stress || s->volume) {
         if (!c->tmp) HIPCHK(hipMalloc((void**)&c->tmp, 60 * E * sizeof(double)));
     }
@@ -4232,24 +4237,24 @@ extern "C" int snh_download_state(snh_context* c, snh_state* s) {
             HIPCHK(hipGetLastError());
             src = c->tmp;
         }
-        if ((rc = download_rows(c, src, s->stress, E, XF_STRESS))) return rc;
+        if ((rc = download_rows(c, land, src, s->stress, E, XF_STRESS))) return rc;
     }
     if (s->volume) {
         StepArgs a = make_args(c);
         hipLaunchKernelGGL(k_volumes, dim3((c->E + 127) / 128), dim3(128), 0, c->stream, a, c->tmp);
         HIPCHK(hipGetLastError());
-        if ((rc = download_rows(c, c->tmp, s->volume, E, XF_TET))) return rc;
+        if ((rc = download_rows(c, land, c->tmp, s->volume, E, XF_TET))) return rc;
     }
     if (s->plastic_strain) {
-        if (c->ps) {
-            if ((rc = download_rows(c, c->ps, s->plastic_strain, E, XF_TET))) return rc;
+        if (ps) {
+            if ((rc = download_rows(c, land, c->ps, s->plastic_strain, E, XF_TET))) return rc;
         } else {
             memset(s->plastic_strain, 0, 10 * E * sizeof(double));
         }
     }
     if (s->viscosity) {
-        if (c->visc) {
-            if ((rc = download_rows(c, c->visc, s->viscosity, E, XF_TET))) return rc;
+        if (visc) {
+            if ((rc = download_rows(c, land, c->visc, s->viscosity, E, XF_TET))) return rc;
         } else {
             /* linear law: the viscosity is the clamped reference viscosity */
             std::vector<double> rv;
@@ -4274,6 +4279,7 @@ extern "C" int snh_download_state(snh_context* c, snh_state* s) {
             }
         }
     }
+    HIPCHK(land.finish());
     return SNH_OK;
 }
 
