@@ -141,9 +141,10 @@ __device__ void tred2_3(double d[3], double e[3], double V[3][3]) {
             }
         } else {
             double f, g, hh;
+            const snh_recip rscale = snh_recip_make(scale);
 #pragma unroll
             for (int k = 0; k < i; k++) {
-                d[k] /= scale;
+                d[k] = snh_quot(d[k], rscale);
                 h += d[k] * d[k];
             }
             f = d[i - 1];
@@ -152,6 +153,7 @@ __device__ void tred2_3(double d[3], double e[3], double V[3][3]) {
             e[i] = scale * g;
             h = h - f * g;
             d[i - 1] = f - g;
+            const snh_recip rh = snh_recip_make(h);
 #pragma unroll
             for (int j = 0; j < i; j++) e[j] = 0.0;
 #pragma unroll
@@ -169,10 +171,10 @@ __device__ void tred2_3(double d[3], double e[3], double V[3][3]) {
             f = 0.0;
 #pragma unroll
             for (int j = 0; j < i; j++) {
-                e[j] /= h;
+                e[j] = snh_quot(e[j], rh);
                 f += e[j] * d[j];
             }
-            hh = f / (h + h);
+            hh = 0.5 * snh_quot(f, rh);   /* f / (h + h) */
 #pragma unroll
             for (int j = 0; j < i; j++) e[j] -= hh * d[j];
 #pragma unroll
@@ -194,8 +196,9 @@ __device__ void tred2_3(double d[3], double e[3], double V[3][3]) {
         V[i][i] = 1.0;
         h = d[i + 1];
         if (h != 0.0) {
+            const snh_recip rh = snh_recip_make(h);
 #pragma unroll
-            for (int k = 0; k <= i; k++) d[k] = V[k][i + 1] / h;
+            for (int k = 0; k <= i; k++) d[k] = snh_quot(V[k][i + 1], rh);
 #pragma unroll
             for (int j = 0; j <= i; j++) {
                 g = 0.0;
@@ -268,11 +271,12 @@ __device__ void tql2_3(double d[3], double e[3], double V[3][3]) {
             int guard = 0;
             do {
                 double g = d[l];
-                double p = (d[l + 1] - g) / (2.0 * e[l]);
+                /* |e[l]| >= 1 here: its int abs() is not zero */
+                double p = 0.5 * snh_quot(d[l + 1] - g, snh_recip_make(e[l]));   /* (..) / (2 e[l]) */
                 double r = snh_hypot(p, 1.0);
                 double dl1, h, cc, c2, c3, el1, s, s2;
                 if (p < 0) r = -r;
-                d[l] = e[l] / (p + r);
+                d[l] = snh_quot(e[l], snh_recip_make(p + r));
                 d[l + 1] = e[l] * (p + r);
                 dl1 = d[l + 1];
                 h = g - d[l];
@@ -295,13 +299,14 @@ __device__ void tql2_3(double d[3], double e[3], double V[3][3]) {
                     h = cc * p;
                     r = snh_hypot(p, ei);
                     set3(e, i + 1, s * r);
-                    s = ei / r;
-                    cc = p / r;
+                    const snh_recip rr = snh_recip_make(r);
+                    s = snh_quot(ei, rr);
+                    cc = snh_quot(p, rr);
                     p = cc * di - s * g;
                     set3(d, i + 1, h + s * (cc * g + s * di));
                     rot_cols(V, i, s, cc);
                 }
-                p = -s * s2 * c3 * el1 * e[l] / dl1;
+                p = snh_quot(-s * s2 * c3 * el1 * e[l], snh_recip_make(dl1));
                 e[l] = s * p;
                 d[l] = cc * p;
                 /* the reference loop has no iteration cap; a cap of 64
@@ -375,17 +380,23 @@ __device__ __forceinline__ bool mc_return(const DevMaterial& m, double st[3][3],
     const double a1 = m.lambda + 2.0 * m.mu;
     const double a2 = m.lambda;
     double alam, dep1, dep2, dep3;
-    double anphi = (1.0 + sphi) / (1.0 - sphi);
-    double anpsi = (1.0 + spsi) / (1.0 - spsi);
-    double fs = s[0] - s[2] * anphi + 2 * cohesion * sqrt(anphi);
+    /* the host's values of the table's first angles (the same correctly
+       rounded operations), unless softening has changed them */
+    double anphi = m.anphi0, sqanphi = m.sqanphi0, anpsi = m.anpsi0;
+    if (sphi != m.sphi) {
+        anphi = (1.0 + sphi) / (1.0 - sphi);
+        sqanphi = sqrt(anphi);
+    }
+    if (spsi != m.spsi) anpsi = (1.0 + spsi) / (1.0 - spsi);
+    double fs = s[0] - s[2] * anphi + 2 * cohesion * sqanphi;
     double ft = s[2] - tension_cutoff;
     if (!(fs < 0.0 || ft > 0.0)) return false;
     double aP = sqrt(1.0 + anphi * anphi) + anphi;
-    double sP = tension_cutoff * anphi - 2 * cohesion * sqrt(anphi);
+    double sP = tension_cutoff * anphi - 2 * cohesion * sqanphi;
     double h = s[2] - tension_cutoff + aP * (s[0] - sP);
     if (h < 0.0) {
         if (with_hard)
-            alam = fs / (a1 - a2 * anpsi + a1 * anphi * anpsi - a2 * anphi + 2.0 * sqrt(anphi) * hardening);
+            alam = fs / (a1 - a2 * anpsi + a1 * anphi * anpsi - a2 * anphi + 2.0 * sqanphi * hardening);
         else
             alam = fs / (a1 - a2 * anpsi + a1 * anphi * anpsi - a2 * anphi);
         s[0] -= alam * (a1 - a2 * anpsi);
@@ -419,6 +430,39 @@ __device__ __forceinline__ bool mc_return(const DevMaterial& m, double st[3][3],
     return true;
 }
 
+/* the same return for viscoplastic_BI, which hands the eigen-solver the upper
+   triangle of the tensor alone (viscoplastic_BI/Constitutive.c:246): the
+   solver reads the lower one, whose off-diagonal entries are zero, so its
+   eigenvalues are the diagonal sorted and its eigenvectors unit vectors, and
+   the back-rotation puts each principal stress on the diagonal entry it came
+   from */
+__device__ __forceinline__ bool vp_return(const DevMaterial& m, double st[6], double sphi, double spsi, double coh,
+                                          double tc, double hardening, double& dps) {
+    double s[3] = {st[0], st[1], st[2]};
+    int at[3] = {0, 1, 2};
+#pragma unroll
+    for (int i = 0; i < 2; i++)   /* the solver's ascending sort */
+#pragma unroll
+        for (int j = i + 1; j < 3; j++) {
+            /* selection with strict comparison: the first smallest of the
+               entries from i on goes to i */
+            const bool less = s[j] < s[i];
+            const double si = s[i];
+            const int ai = at[i];
+            s[i] = less ? s[j] : si;
+            s[j] = less ? si : s[j];
+            at[i] = less ? at[j] : ai;
+            at[j] = less ? ai : at[j];
+        }
+    double S[3][3];
+    const double cn[3][3] = {{1.0, 0.0, 0.0}, {0.0, 1.0, 0.0}, {0.0, 0.0, 1.0}};
+    if (!mc_return(m, S, s, cn, sphi, spsi, coh, tc, hardening, true, dps)) return false;
+#pragma unroll
+    for (int c = 0; c < 3; c++) st[c] = at[0] == c ? s[0] : (at[1] == c ? s[1] : s[2]);
+    st[3] = st[4] = st[5] = 0.0;
+    return true;
+}
+
 /* sines/tangent of the softened angles: the host's libm values when the
    angles equal the first table entry (constant-angle tables), the device's
    otherwise */
@@ -446,12 +490,19 @@ __device__ __forceinline__ bool mc_surely_elastic(const DevMaterial& m, const do
     const double p = (st[0] + st[1] + st[2]) * (1.0 / 3.0);
     const double d0 = st[0] - p, d1 = st[1] - p, d2 = st[2] - p;
     const double r2 = d0 * d0 + d1 * d1 + d2 * d2 + 2.0 * (st[3] * st[3] + st[4] * st[4] + st[5] * st[5]);
-    const double r = sqrt(r2 * (2.0 / 3.0));
-    const double anphi = sphi == m.sphi ? m.anphi0 : (1.0 + sphi) / (1.0 - sphi);
+    /* the root from v_rsq_f64's estimate, 2^-23 off at most, kept on the safe
+       side (a zero deviator gives a root of 1e-100, not 0 times infinity) */
+    const double q = fmax(r2 * (2.0 / 3.0), 1e-200);
+    const double r = q * __builtin_amdgcn_rsq(q) * (1.0 + 1e-6);
+    double anphi = m.anphi0, sqanphi = m.sqanphi0;
+    if (sphi != m.sphi) {
+        anphi = (1.0 + sphi) / (1.0 - sphi);
+        sqanphi = sqrt(anphi);
+    }
     const double smin = p - r, smax = p + r;
     const double scale = fabs(p) + r + fabs(cohesion) + fabs(tc);
     const double margin = 64.0 + 1e-9 * scale * (1.0 + anphi);
-    const double fs_lo = smin - smax * anphi + 2.0 * cohesion * (sphi == m.sphi ? m.sqanphi0 : sqrt(anphi));
+    const double fs_lo = smin - smax * anphi + 2.0 * cohesion * sqanphi;
     const double ft_hi = smax - tc;
     return fs_lo > margin && ft_hi < -margin;
 }
@@ -460,7 +511,9 @@ __device__ __forceinline__ bool mc_surely_elastic(const DevMaterial& m, const do
    for a tet that may yield; out of line, so that the registers it needs are
    not reserved across the whole element loop (most tets never call it).
    io[0..5] holds the trial stress; on yield it holds the returned stress and
-   io[6] the plastic strain increment. */
+   io[6] the plastic strain increment.  One copy for each number of waves per
+   SIMD its callers ask for: a copy's registers count towards theirs. */
+template <int WAVES>
 __device__ __noinline__ bool mc_plastic_update(const DevMaterial& m, double* io, double sphi, double spsi,
                                                double coh, double tc) {
     double S[3][3];
@@ -481,10 +534,11 @@ __device__ __noinline__ bool mc_plastic_update(const DevMaterial& m, double* io,
    caller's st stays in registers instead of living in scratch memory for
    the whole kernel (an array whose address reaches an out-of-line call
    cannot be promoted). */
+template <int WAVES>
 __device__ __forceinline__ bool mc_plastic_step(const DevMaterial& m, double st[6], double sphi, double spsi,
                                                 double coh, double tc, double& dps) {
     double io[7] = {st[0], st[1], st[2], st[3], st[4], st[5], 0.0};
-    if (!mc_plastic_update(m, io, sphi, spsi, coh, tc)) return false;
+    if (!mc_plastic_update<WAVES>(m, io, sphi, spsi, coh, tc)) return false;
 #pragma unroll
     for (int c = 0; c < 6; c++) st[c] = io[c];
     dps = io[6];
@@ -633,6 +687,23 @@ __device__ __forceinline__ void store_density_at(const StepArgs& a, const DevMat
     store_density(a, m, nd, t, e);
 }
 
+/* base[off / 8] for a uniform base and a per-lane byte offset below 4 GB (a
+   row of E or N doubles: device memory holds fewer than 2^29 elements): the
+   load takes its base from scalar registers and its offset from one vector
+   register, so a row costs no vector address arithmetic */
+typedef const __attribute__((address_space(1))) char* gbase;   /* uniform, in global memory */
+__device__ __forceinline__ gbase row_base(const double* p) { return (gbase)(uintptr_t)p; }
+__device__ __forceinline__ double ld_row(gbase base, size_t row, uint32_t off) {
+    gbase b = base + 8 * row;
+    asm("" : "+s"(b), "+v"(off));   /* keeps the row's base scalar and the offset 32 bits wide */
+    return *(const __attribute__((address_space(1))) double*)(b + off);
+}
+__device__ __forceinline__ void st_row(double* p, size_t row, uint32_t off, double v) {
+    __attribute__((address_space(1))) char* b = (__attribute__((address_space(1))) char*)(uintptr_t)p + 8 * row;
+    asm("" : "+s"(b), "+v"(off));
+    *(__attribute__((address_space(1))) double*)(b + off) = v;
+}
+
 /* softened parameters carried along the tets of an element: the reference
    declares them once per element (plastic_BI/Constitutive.c:78-81,
    viscoplastic_BI/Constitutive.c:115-119) */
@@ -640,29 +711,155 @@ struct Soft {
     double phi, psi, coh, hard;
 };
 
-/* TW = false: one 64-lane block holds 6 elements x 10 tets.
-   TW = true ("tet per wave"): a 640-thread block holds 64 elements, wave w
-   taking tet w of all of them, so every stress and node load of a wave is
-   over 64 consecutive elements. */
-template <int RSET, bool TW, bool MM>
+/* the parameters of the segment that holds plastic strain ps, if one does */
+__device__ __forceinline__ bool soften_own(const DevMaterial& m, const double ps, Soft& o) {
+    bool matched = false;
+    for (uint32_t i = 0; i < m.nseg; i++) {
+        const double pl1 = m.plstrain[i], pl2 = m.plstrain[i + 1];
+        if (ps >= pl1 && ps <= pl2) {
+            const double tgf = m.tgf[i];
+            const double tgd = m.tgd[i];
+            const double tgc = m.tgc[i];
+            o.phi = m.fa[i] + tgf * (ps - pl1);
+            o.psi = m.da[i] + tgd * (ps - pl1);
+            o.coh = m.coh[i] + tgc * (ps - pl1);
+            o.hard = tgc;
+            matched = true;
+        }
+    }
+    return matched;
+}
+
+/* The parameters of tet t: its own segment's when its plastic strain lies in
+   one and the angle is not negative; otherwise those carried from the tets
+   before it, in order.  pst[q * stride] is the stored plastic strain of the
+   element's tet q (LDS); ps, this tet's, is reset with a negative one. */
+__device__ __forceinline__ Soft soften_tet(const DevMaterial& m, const bool is_pl, const int t, const double* pst,
+                                           const int stride, double& ps) {
+    Soft sp = {0.0, 0.0, 0.0, 0.0};
+    if (soften_own(m, ps, sp) && sp.phi >= 0.0) return sp;
+    sp = {is_pl ? 30.0 : 0.0, 0.0, is_pl ? 30.0e6 : 0.0, 0.0};   /* plastic_BI :78-80 defaults */
+    for (int q = 0; q <= t; q++) {
+        const double psq = pst[q * stride];
+        (void)soften_own(m, psq, sp);
+        if (!(sp.phi >= 0.0) && psq < 0.0) {
+            /* negative plastic strain is reset (plastic_BI :143-151) */
+            sp.phi = m.fa[0];
+            sp.psi = m.da[0];
+            sp.coh = m.coh[0];
+            if (q == t) ps = 0.0;
+        }
+    }
+    return sp;
+}
+
+/* what a tet brings to its material's law */
+struct TetLaw {
+    int t, e;          /* tet and element                            */
+    bool active;       /* stores are for an element of the mesh      */
+    bool is_pl, is_vp;
+    double V, dt;
+    double rvisc;      /* the element's reference viscosity          */
+    double ps_in;      /* stored plastic strain                      */
+};
+
+/* the material's law on the rotated stress st with strain sn, and the tet's
+   plastic strain; nd: the tet's four nodes */
+template <int RSET, int WAVES>
+__device__ __forceinline__ void tet_law(const StepArgs& a, const DevMaterial& m, const TetLaw& k, const int nd[4],
+                                        const Soft& sp, double ps, const double sn[6], double st[6]) {
+    const size_t E = (size_t)a.E;
+    if ((RSET & RS_PLASTIC) && k.is_pl) {
+        double trace_strain = sn[0] + sn[1] + sn[2];
+        st[0] += (2.0 * m.mu) * sn[0] + m.lambda * (trace_strain);
+        st[1] += (2.0 * m.mu) * sn[1] + m.lambda * (trace_strain);
+        st[2] += (2.0 * m.mu) * sn[2] + m.lambda * (trace_strain);
+        st[3] += (2.0 * m.mu) * sn[3];
+        st[4] += (2.0 * m.mu) * sn[4];
+        st[5] += (2.0 * m.mu) * sn[5];
+        const double coh = a.cohoff ? sp.coh + a.cohoff[k.e] : sp.coh;
+        double sphi, spsi, dps = 0.0;
+        angle_terms(m, sp.phi, sp.psi, sphi, spsi);
+        bool changed = false;
+        /* the bound takes the tension cut-off as a product with 1 / tan phi
+           (its margin covers the rounding); the return divides */
+        const bool derived = sp.phi > 0.0 && m.ten_off == 0.0;
+        double tc = m.ten_off;
+        if (derived) tc = sp.phi == m.fa[0] ? coh * m.rtanphi0 : coh / tan_phi(m, sp.phi);
+        if (!mc_surely_elastic(m, st, sphi, coh, tc)) {
+            if (derived) tc = coh / tan_phi(m, sp.phi);
+            if (mc_plastic_step<WAVES>(m, st, sphi, spsi, coh, tc, dps)) {
+                ps = ps + dps;
+                changed = true;
+            }
+        }
+        /* in place, an unchanged value need not be stored */
+        if (k.active && (changed || a.ps_out != a.ps || ps != k.ps_in)) a.ps_out[(size_t)k.t * E + k.e] = ps;
+    } else if ((RSET & RS_VISCOPLASTIC) && k.is_vp) {
+        add_thermal_stress(a, st, k.t, k.e);
+        double trace_strain = sn[0] + sn[1] + sn[2];
+        double d0, d1, d2;
+        devstrain(sn, trace_strain, d0, d1, d2);
+        double visc = viscosity_of(m, k.rvisc, d0, d1, d2, sn, k.dt, tet_temp(a, m, nd));
+        if (a.visc && k.active) a.visc[(size_t)k.t * E + k.e] = visc;
+        maxwell_update(m, st, sn, trace_strain, visc, k.dt);
+        const double coh = a.cohoff ? sp.coh + a.cohoff[k.e] : sp.coh;
+        double tc = m.ten_off;
+        if (sp.phi > 0.0 && tc == 0.0) tc = coh / tan_phi(m, sp.phi);
+        double sphi, spsi, dps = 0.0;
+        angle_terms(m, sp.phi, sp.psi, sphi, spsi);
+        if (vp_return(m, st, sphi, spsi, coh, tc, sp.hard, dps)) ps = ps + dps;
+        if (k.active) a.ps_out[(size_t)k.t * E + k.e] = ps;
+    } else if ((RSET & RS_MAXWELL) && (m.rheology & SNH_RHEOLOGY_MAXWELL)) {
+        /* trace strain from the volume ratio (maxwell/Constitutive.c:113) */
+        double Xp[4][3];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            Xp[q][0] = a.xp[nd[q]];
+            Xp[q][1] = a.xp[a.N + nd[q]];
+            Xp[q][2] = a.xp[2 * a.N + nd[q]];
+        }
+        double old_volume = tet_volume(Xp[0], Xp[1], Xp[2], Xp[3]);
+        double trace_strain = k.V / old_volume - 1.0;
+        add_thermal_stress(a, st, k.t, k.e);
+        double d0, d1, d2;
+        devstrain(sn, trace_strain, d0, d1, d2);
+        double visc = viscosity_of(m, k.rvisc, d0, d1, d2, sn, k.dt, tet_temp(a, m, nd));
+        if (a.visc && k.active) a.visc[(size_t)k.t * E + k.e] = visc;
+        maxwell_update(m, st, sn, trace_strain, visc, k.dt);
+    } else if ((RSET & RS_ELASTIC) && (m.rheology & SNH_RHEOLOGY_ELASTIC)) {
+        const double a2 = m.lambda;
+        const double sh2 = 2.0 * m.mu;
+        double trace_strain = sn[0] + sn[1] + sn[2];
+        st[0] += sh2 * sn[0] + a2 * (trace_strain);
+        st[1] += sh2 * sn[1] + a2 * (trace_strain);
+        st[2] += sh2 * sn[2] + a2 * (trace_strain);
+        st[3] += sh2 * sn[3];
+        st[4] += sh2 * sn[4];
+        st[5] += sh2 * sn[5];
+    }
+}
+
+/* One lane per tet: a 64-lane block holds 6 elements x 10 tets (lanes 60..63
+   carry no tet: they mirror tet 0 of element slot 0 but never write LDS or
+   memory).  A lane's place in the ten tets' rows of a component must fit 32
+   bits of byte offset: at most LANE_MOST_ELEMENTS elements. */
+#define LANE_MOST_ELEMENTS 53687091
+template <int RSET, bool MM>
 __device__ __forceinline__ void elem_pass(StepArgs a, const int blk, const int nblk) {
-    constexpr int NE = TW ? 64 : EPW;       /* elements per block */
-    constexpr int NT = TW ? NTET + 1 : NTET; /* padded against LDS bank conflicts */
-    __shared__ double sh_a[NE][NT];
-    __shared__ double sh_b[NE][NT];
-    __shared__ double sh_c[NE][NT];   /* the stress-trace sums */
-    __shared__ double sh_sp[NE][NT][5];   /* matched, phi, psi, coh, hard */
-    __shared__ double sh_ps[NE][NT];
+    __shared__ double sh_a[EPW][NTET];
+    __shared__ double sh_b[EPW][NTET];
+    __shared__ double sh_c[EPW][NTET];   /* the stress-trace sums */
+    __shared__ double sh_ps[EPW][NTET];
     const int lane = threadIdx.x;
-    /* (tet-per-lane) lanes 60..63 carry no tet: they mirror tet 0 of element
-       slot 0 but never write LDS or memory */
-    const bool in_wave = TW || lane < EPW * NTET;
-    const int le = TW ? (lane & 63) : (in_wave ? lane / NTET : 0);
-    const int t = TW ? (lane >> 6) : (in_wave ? lane - le * NTET : 0);
-    const int e = xcd_block(blk, nblk) * NE + le;
+    const bool in_wave = lane < EPW * NTET;
+    const int le = in_wave ? lane / NTET : 0;
+    const int t = in_wave ? lane - le * NTET : 0;
+    const int e = xcd_block(blk, nblk) * EPW + le;
     const bool active = in_wave && e < a.E;
     const size_t E = (size_t)a.E;
     const int ec = active ? e : 0;
+    const uint32_t to = 8u * ((uint32_t)t * (uint32_t)a.E + (uint32_t)ec);   /* of the tet, in a component's rows */
     int ei, ej, ek;
     elem_ijk(a, ec, ei, ej, ek);
     const double dt = a.scal->dt;
@@ -675,18 +872,24 @@ __device__ __forceinline__ void elem_pass(StepArgs a, const int blk, const int n
        laws the same order measured 1-3 % slower). */
     constexpr bool kEarly = RSET == RS_MAXWELL;
     double st[6];
-    double rvisc_e = 0.0;
     if constexpr (kEarly) {
 #pragma unroll
-        for (int c = 0; c < 6; c++) st[c] = active ? a.stress[((size_t)c * NTET + t) * E + ec] : 0.0;
-        rvisc_e = a.refvisc ? a.refvisc[ec] : m.refvisc;
+        for (int c = 0; c < 6; c++) st[c] = ld_row(row_base(a.stress), (size_t)c * NTET * E, to);
     }
+    TetLaw law;
+    law.t = t;
+    law.e = ec;
+    law.active = active;
+    law.dt = dt;
+    law.is_pl = (RSET & RS_PLASTIC) && (m.rheology & SNH_RHEOLOGY_PLASTIC);
+    law.is_vp = (RSET & RS_VISCOPLASTIC) && (m.rheology & SNH_RHEOLOGY_VISCOPLASTIC);
+    law.rvisc = (RSET & (RS_MAXWELL | RS_VISCOPLASTIC)) ? (a.refvisc ? a.refvisc[ec] : m.refvisc) : 0.0;
     /* the plastic laws' stored plastic strain, likewise ahead of the
        kinematics (1.6 % off the Mohr-Coulomb pass) */
-    const bool is_pl = (RSET & RS_PLASTIC) && (m.rheology & SNH_RHEOLOGY_PLASTIC);
-    const bool is_vp = (RSET & RS_VISCOPLASTIC) && (m.rheology & SNH_RHEOLOGY_VISCOPLASTIC);
+    const bool soft = law.is_pl || law.is_vp;
     double ps = 0.0;
-    if ((RSET & (RS_PLASTIC | RS_VISCOPLASTIC)) && (is_pl || is_vp) && active) ps = a.ps[(size_t)t * E + ec];
+    if ((RSET & (RS_PLASTIC | RS_VISCOPLASTIC)) && soft) ps = ld_row(row_base(a.ps), 0, to);
+    law.ps_in = ps;
 
     /* kinematics of this lane's tet (UpdateElement.c:84-219, StrainRate.c:65-184) */
     int nd[4];
@@ -694,19 +897,20 @@ __device__ __forceinline__ void elem_pass(StepArgs a, const int blk, const int n
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         nd[q] = hex_node_index(a, ei, ej, ek, tet_node(t, q));
-        Xt[q][0] = a.xc[nd[q]];
-        Xt[q][1] = a.xc[a.N + nd[q]];
-        Xt[q][2] = a.xc[2 * a.N + nd[q]];
-        Ut[q][0] = a.v[nd[q]];
-        Ut[q][1] = a.v[a.N + nd[q]];
-        Ut[q][2] = a.v[2 * a.N + nd[q]];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            Xt[q][d] = ld_row(row_base(a.xc), (size_t)d * (size_t)a.N, 8u * (uint32_t)nd[q]);
+            Ut[q][d] = ld_row(row_base(a.v), (size_t)d * (size_t)a.N, 8u * (uint32_t)nd[q]);
+        }
     }
     TetKin k;
     tet_kinematics(Xt, Ut, k);
+    law.V = k.V;
     const double trace = snh_div3(k.sr[0] + k.sr[1] + k.sr[2]);
     if (in_wave) {
         sh_a[le][t] = k.V;
         sh_b[le][t] = trace * k.V;
+        if (RSET & (RS_PLASTIC | RS_VISCOPLASTIC)) sh_ps[le][t] = ps;
     }
     __syncthreads();
     double evol = 0.0, partial = 0.0;
@@ -723,7 +927,7 @@ __device__ __forceinline__ void elem_pass(StepArgs a, const int blk, const int n
     /* rotation of the stored stress, strain (Stress.c:71-82) */
     if constexpr (!kEarly) {
 #pragma unroll
-        for (int c = 0; c < 6; c++) st[c] = active ? a.stress[((size_t)c * NTET + t) * E + ec] : 0.0;
+        for (int c = 0; c < 6; c++) st[c] = ld_row(row_base(a.stress), (size_t)c * NTET * E, to);
     }
     rotate_stress(st, k.w, dt_rot);
     double sn[6];
@@ -733,137 +937,8 @@ __device__ __forceinline__ void elem_pass(StepArgs a, const int blk, const int n
     for (int c = 3; c < 6; c++) sn[c] = k.sr[c] * dt;
 
     Soft sp = {0.0, 0.0, 0.0, 0.0};
-    if (RSET & (RS_PLASTIC | RS_VISCOPLASTIC)) {
-        /* own segment match, then resolve the carried parameters in tet order */
-        double matched = 0.0;
-        Soft own = {0.0, 0.0, 0.0, 0.0};
-        if (is_pl || is_vp) {
-            for (uint32_t i = 0; i < m.nseg; i++) {
-                const double pl1 = m.plstrain[i], pl2 = m.plstrain[i + 1];
-                if (ps >= pl1 && ps <= pl2) {
-                    const double tgf = m.tgf[i];
-                    const double tgd = m.tgd[i];
-                    const double tgc = m.tgc[i];
-                    own.phi = m.fa[i] + tgf * (ps - pl1);
-                    own.psi = m.da[i] + tgd * (ps - pl1);
-                    own.coh = m.coh[i] + tgc * (ps - pl1);
-                    own.hard = tgc;
-                    matched = 1.0;
-                }
-            }
-        }
-        if (in_wave) {
-            sh_sp[le][t][0] = matched;
-            sh_sp[le][t][1] = own.phi;
-            sh_sp[le][t][2] = own.psi;
-            sh_sp[le][t][3] = own.coh;
-            sh_sp[le][t][4] = own.hard;
-            sh_ps[le][t] = ps;
-        }
-        __syncthreads();
-        if ((is_pl || is_vp) && matched != 0.0 && own.phi >= 0.0) {
-            /* the scan below ends with this tet's own parameters whenever its
-               plastic strain lies in a segment and the angle is not negative */
-            sp = own;
-        } else if (is_pl || is_vp) {
-            sp.phi = is_pl ? 30.0 : 0.0;   /* plastic_BI :78-80 defaults */
-            sp.coh = is_pl ? 30.0e6 : 0.0;
-            for (int q = 0; q <= t; q++) {
-                if (sh_sp[le][q][0] != 0.0) {
-                    sp.phi = sh_sp[le][q][1];
-                    sp.psi = sh_sp[le][q][2];
-                    sp.coh = sh_sp[le][q][3];
-                    sp.hard = sh_sp[le][q][4];
-                }
-                if (!(sp.phi >= 0.0) && sh_ps[le][q] < 0.0) {
-                    /* negative plastic strain is reset (plastic_BI :143-151) */
-                    sp.phi = m.fa[0];
-                    sp.psi = m.da[0];
-                    sp.coh = m.coh[0];
-                    if (q == t) ps = 0.0;
-                }
-            }
-        }
-    }
-
-    if (is_pl) {
-        double trace_strain = sn[0] + sn[1] + sn[2];
-        double S[3][3];
-        st[0] += (2.0 * m.mu) * sn[0] + m.lambda * (trace_strain);
-        st[1] += (2.0 * m.mu) * sn[1] + m.lambda * (trace_strain);
-        st[2] += (2.0 * m.mu) * sn[2] + m.lambda * (trace_strain);
-        st[3] += (2.0 * m.mu) * sn[3];
-        st[4] += (2.0 * m.mu) * sn[4];
-        st[5] += (2.0 * m.mu) * sn[5];
-        S[0][0] = st[0]; S[1][1] = st[1]; S[2][2] = st[2];
-        S[0][1] = S[1][0] = st[3];
-        S[0][2] = S[2][0] = st[4];
-        S[1][2] = S[2][1] = st[5];
-        const double coh = a.cohoff ? sp.coh + a.cohoff[ec] : sp.coh;
-        double tc = m.ten_off;
-        if (sp.phi > 0.0 && tc == 0.0) tc = coh / tan_phi(m, sp.phi);
-        double sphi, spsi, dps = 0.0;
-        angle_terms(m, sp.phi, sp.psi, sphi, spsi);
-        bool changed = false;
-        if (!mc_surely_elastic(m, st, sphi, coh, tc) && mc_plastic_step(m, st, sphi, spsi, coh, tc, dps)) {
-            ps = ps + dps;
-            changed = true;
-        }
-        /* in place, an unchanged value need not be stored */
-        if (active && (changed || a.ps_out != a.ps || ps != sh_ps[le][t])) a.ps_out[(size_t)t * E + ec] = ps;
-    } else if (is_vp) {
-        add_thermal_stress(a, st, t, ec);
-        double trace_strain = sn[0] + sn[1] + sn[2];
-        double d0, d1, d2;
-        devstrain(sn, trace_strain, d0, d1, d2);
-        double rvisc = kEarly ? rvisc_e : (a.refvisc ? a.refvisc[ec] : m.refvisc);
-        double visc = viscosity_of(m, rvisc, d0, d1, d2, sn, dt, tet_temp(a, m, nd));
-        if (a.visc && active) a.visc[(size_t)t * E + ec] = visc;
-        maxwell_update(m, st, sn, trace_strain, visc, dt);
-        /* unsymmetrised: the lower triangle is zero (viscoplastic_BI :246) */
-        double S[3][3] = {{st[0], st[3], st[4]}, {0.0, st[1], st[5]}, {0.0, 0.0, st[2]}};
-        double d3[3], cn[3][3];
-        principal_stresses(S, d3, cn);
-        const double coh = a.cohoff ? sp.coh + a.cohoff[ec] : sp.coh;
-        double tc = m.ten_off;
-        if (sp.phi > 0.0 && tc == 0.0) tc = coh / tan_phi(m, sp.phi);
-        double sphi, spsi, dps = 0.0;
-        angle_terms(m, sp.phi, sp.psi, sphi, spsi);
-        if (mc_return(m, S, d3, cn, sphi, spsi, coh, tc, sp.hard, true, dps)) {
-            ps = ps + dps;
-            st[0] = S[0][0]; st[1] = S[1][1]; st[2] = S[2][2];
-            st[3] = S[0][1]; st[4] = S[0][2]; st[5] = S[1][2];
-        }
-        if (active) a.ps_out[(size_t)t * E + ec] = ps;
-    } else if ((RSET & RS_MAXWELL) && (m.rheology & SNH_RHEOLOGY_MAXWELL)) {
-        /* trace strain from the volume ratio (maxwell/Constitutive.c:113) */
-        double Xp[4][3];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            Xp[q][0] = a.xp[nd[q]];
-            Xp[q][1] = a.xp[a.N + nd[q]];
-            Xp[q][2] = a.xp[2 * a.N + nd[q]];
-        }
-        double old_volume = tet_volume(Xp[0], Xp[1], Xp[2], Xp[3]);
-        double trace_strain = k.V / old_volume - 1.0;
-        add_thermal_stress(a, st, t, ec);
-        double d0, d1, d2;
-        devstrain(sn, trace_strain, d0, d1, d2);
-        double rvisc = kEarly ? rvisc_e : (a.refvisc ? a.refvisc[ec] : m.refvisc);
-        double visc = viscosity_of(m, rvisc, d0, d1, d2, sn, dt, tet_temp(a, m, nd));
-        if (a.visc && active) a.visc[(size_t)t * E + ec] = visc;
-        maxwell_update(m, st, sn, trace_strain, visc, dt);
-    } else if ((RSET & RS_ELASTIC) && (m.rheology & SNH_RHEOLOGY_ELASTIC)) {
-        const double a2 = m.lambda;
-        const double sh2 = 2.0 * m.mu;
-        double trace_strain = sn[0] + sn[1] + sn[2];
-        st[0] += sh2 * sn[0] + a2 * (trace_strain);
-        st[1] += sh2 * sn[1] + a2 * (trace_strain);
-        st[2] += sh2 * sn[2] + a2 * (trace_strain);
-        st[3] += sh2 * sn[3];
-        st[4] += sh2 * sn[4];
-        st[5] += sh2 * sn[5];
-    }
+    if ((RSET & (RS_PLASTIC | RS_VISCOPLASTIC)) && soft) sp = soften_tet(m, law.is_pl, t, sh_ps[le], 1, ps);
+    tet_law<RSET, 1>(a, m, law, nd, sp, ps, sn, st);
 
     /* stress trace averaging (Stress.c:87-137) */
     const double tr = snh_div3(st[0] + st[1] + st[2]);
@@ -879,14 +954,177 @@ __device__ __forceinline__ void elem_pass(StepArgs a, const int blk, const int n
     st[2] += -1.0 * tr + avgTrace;
     if (active) {
 #pragma unroll
-        for (int c = 0; c < 6; c++) a.stress_out[((size_t)c * NTET + t) * E + ec] = st[c];
+        for (int c = 0; c < 6; c++) st_row(a.stress_out, (size_t)c * NTET * E, to, st[c]);
         if (a.tpre) store_density(a, m, nd, t, ec);
     }
 }
 
+/* "Tet per wave": the waves of a block share 64 elements, each taking one or
+   two of the ten tets of all of them, so every load and store of a wave is
+   over 64 consecutive elements of one row and everything that depends on the
+   tet is scalar.  Which, by the law, at 256x64x128 elements:
+   - elastic, Maxwell: five waves, tets w and w + 5 one after the other; what
+     the second phase needs of the first tet waits in LDS.  At 96 registers and
+     41 KB three blocks share a CU and cover each other's loads and barriers:
+     660 and 833 us, against 729 and 900 us with ten waves (one block a CU) and
+     870 and 1020 us with ten waves and vector addresses;
+   - the plastic laws: ten waves of one tet, up to 168 registers: 884 us
+     Mohr-Coulomb and 1026 us visco-plastic, against 920 and 1075 us with five
+     (their return diverges, and a wave then does it for both its tets) and
+     1160 and 1445 us with ten waves held to 96 registers.
+   What bounds it now is the wait for its loads and barriers: at 884 us the
+   Mohr-Coulomb pass issues VALU instructions 35 % of the time and moves 2.4 GB
+   at 2.7 TB/s. */
+__host__ __device__ constexpr int tw_waves(int rset) {
+    return (rset & (RS_PLASTIC | RS_VISCOPLASTIC)) ? 10 : 5;
+}
+__host__ __device__ constexpr int tw_occupancy(int rset) {   /* waves per SIMD the registers leave room for */
+    return (rset & (RS_PLASTIC | RS_VISCOPLASTIC)) ? 3 : 5;
+}
+template <int RSET, bool MM>
+__device__ __forceinline__ void elem_pass_tw(StepArgs a, const int blk, const int nblk) {
+    constexpr int W = tw_waves(RSET), U = NTET / W;
+    constexpr bool kSoft = (RSET & (RS_PLASTIC | RS_VISCOPLASTIC)) != 0;
+    __shared__ double sh_a[NTET][64];
+    __shared__ double sh_b[NTET][64];
+    __shared__ double sh_c[NTET][64];          /* the stress-trace sums */
+    __shared__ double sh_ps[kSoft ? NTET : 1][64];
+    __shared__ double sh_k[U > 1 ? 10 : 1][U > 1 ? 64 * W : 1];      /* strain rate, spin and trace of tet w */
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int e = xcd_block(blk, nblk) * 64 + lane;
+    const bool active = e < a.E;
+    const size_t E = (size_t)a.E;
+    const int ec = active ? e : a.E - 1;
+    const uint32_t eo = 8u * (uint32_t)ec;
+    /* the element's lowest node: with e = ei + EI (ej + EJ ek) it is
+       ei + I (ej + J ek) = e + e / EI + I ek */
+    const int eq = (int)fastdiv((uint32_t)ec, a.dEI);
+    const int n0 = ec + eq + a.I * (int)fastdiv((uint32_t)eq, a.dEJ);
+    const uint32_t no = 8u * (uint32_t)n0;
+    const double dt = a.scal->dt;
+    const double dt_rot = a.scal->dt_rot;
+    const DevMaterial& m = mat_of<MM>(a, ec);
+    TetLaw law;
+    law.e = ec;
+    law.active = active;
+    law.dt = dt;
+    law.is_pl = (RSET & RS_PLASTIC) && (m.rheology & SNH_RHEOLOGY_PLASTIC);
+    law.is_vp = (RSET & RS_VISCOPLASTIC) && (m.rheology & SNH_RHEOLOGY_VISCOPLASTIC);
+    law.rvisc = (RSET & (RS_MAXWELL | RS_VISCOPLASTIC)) ? (a.refvisc ? a.refvisc[ec] : m.refvisc) : 0.0;
+    const bool soft = kSoft && (law.is_pl || law.is_vp);
+
+    /* the node at corner h of an element, relative to its lowest one */
+    auto corner = [&](int h) { return ((h ^ (h >> 1)) & 1) + a.I * (((h >> 1) & 1) + a.J * (h >> 2)); };
+    /* kinematics (UpdateElement.c:84-219, StrainRate.c:65-184) */
+    TetKin k;
+    double trace = 0.0;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const int t = w + W * u;
+        double Xt[4][3], Ut[4][3];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const size_t c = (size_t)corner(tet_node(t, q));
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                Xt[q][d] = ld_row(row_base(a.xc), c + (size_t)d * (size_t)a.N, no);
+                Ut[q][d] = ld_row(row_base(a.v), c + (size_t)d * (size_t)a.N, no);
+            }
+        }
+        if constexpr (kSoft) sh_ps[t][lane] = soft ? ld_row(row_base(a.ps), (size_t)t * E, eo) : 0.0;
+        tet_kinematics(Xt, Ut, k);
+        trace = snh_div3(k.sr[0] + k.sr[1] + k.sr[2]);
+        sh_a[t][lane] = k.V;
+        sh_b[t][lane] = trace * k.V;
+        if (U > 1 && u == 0) {
+#pragma unroll
+            for (int c = 0; c < 6; c++) sh_k[c][threadIdx.x] = k.sr[c];
+#pragma unroll
+            for (int c = 0; c < 3; c++) sh_k[6 + c][threadIdx.x] = k.w[c];
+            sh_k[9][threadIdx.x] = trace;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    /* the stress of the tet that comes first in the second phase */
+    double st[6];
+#pragma unroll
+    for (int c = 0; c < 6; c++) st[c] = ld_row(row_base(a.stress), (size_t)(c * NTET + w + W * (U - 1)) * E, eo);
+    __syncthreads();
+    double evol = 0.0, partial = 0.0;
+#pragma unroll
+    for (int q = 0; q < NTET; q++) {
+        evol += sh_a[q][lane];        /* UpdateElement.c:141 */
+        partial += sh_b[q][lane];     /* StrainRate.c:281 */
+    }
+    evol *= 0.5;                          /* UpdateElement.c:267-268 */
+    const double elemVolume = 2.0 * evol; /* StrainRate.c:57, Stress.c:68 */
+    const snh_recip rEV = snh_recip_make(elemVolume);
+    const double srcorr = snh_quot(partial, rEV);
+
+    double diag[U][3], tr[U];
+#pragma unroll
+    for (int u = U - 1; u >= 0; u--) {
+        const int t = w + W * u;
+        double sn_[6];
+        if (U > 1 && u == 0) {
+#pragma unroll
+            for (int c = 0; c < 6; c++) st[c] = ld_row(row_base(a.stress), (size_t)(c * NTET + t) * E, eo);
+#pragma unroll
+            for (int c = 0; c < 6; c++) k.sr[c] = sh_k[c][threadIdx.x];
+#pragma unroll
+            for (int c = 0; c < 3; c++) k.w[c] = sh_k[6 + c][threadIdx.x];
+            trace = sh_k[9][threadIdx.x];
+            k.V = sh_a[t][lane];
+        }
+        /* rotation of the stored stress, strain (Stress.c:71-82) */
+        rotate_stress(st, k.w, dt_rot);
+#pragma unroll
+        for (int c = 0; c < 3; c++) sn_[c] = (k.sr[c] + (-1.0 * trace + srcorr)) * dt;
+#pragma unroll
+        for (int c = 3; c < 6; c++) sn_[c] = k.sr[c] * dt;
+        law.t = t;
+        law.V = k.V;
+        int nd[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) nd[q] = n0 + corner(tet_node(t, q));
+        Soft sp = {0.0, 0.0, 0.0, 0.0};
+        double ps = 0.0;
+        if constexpr (kSoft) {
+            law.ps_in = ps = sh_ps[t][lane];
+            if (soft) sp = soften_tet(m, law.is_pl, t, &sh_ps[0][lane], 64, ps);
+        }
+        tet_law<RSET, tw_occupancy(RSET)>(a, m, law, nd, sp, ps, sn_, st);
+        /* stress trace averaging (Stress.c:87-137) */
+        tr[u] = snh_div3(st[0] + st[1] + st[2]);
+        sh_c[t][lane] = tr[u] * k.V;
+#pragma unroll
+        for (int c = 0; c < 3; c++) diag[u][c] = st[c];
+        if (active) {
+#pragma unroll
+            for (int c = 3; c < 6; c++) st_row(a.stress_out, (size_t)(c * NTET + t) * E, eo, st[c]);
+            if (a.tpre) store_density(a, m, nd, t, ec);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    double pst = 0.0;
+#pragma unroll
+    for (int q = 0; q < NTET; q++) pst += sh_c[q][lane];
+    const double avgTrace = snh_quot(pst, rEV);
+    if (active) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+                st_row(a.stress_out, (size_t)(c * NTET + w + W * u) * E, eo, diag[u][c] + (-1.0 * tr[u] + avgTrace));
+    }
+}
+
 template <int RSET, bool TW, bool MM>
-__global__ void __launch_bounds__(TW ? 640 : 64) k_elem(StepArgs a) {
-    elem_pass<RSET, TW, MM>(a, (int)blockIdx.x, (int)gridDim.x);
+__global__ void __launch_bounds__(TW ? 64 * tw_waves(RSET) : 64, TW ? tw_occupancy(RSET) : 1) k_elem(StepArgs a) {
+    if constexpr (TW) elem_pass_tw<RSET, MM>(a, (int)blockIdx.x, (int)gridDim.x);
+    else elem_pass<RSET, MM>(a, (int)blockIdx.x, (int)gridDim.x);
 }
 
 /* --------------------------------------------------------------------------
@@ -1040,7 +1278,7 @@ __global__ void __launch_bounds__(ELEM_BLOCK) k_elem_seq(StepArgs a) {
             double sphi, spsi;
             angle_terms(m, pphi, ppsi, sphi, spsi);
             double dps = 0.0;
-            if (!mc_surely_elastic(m, st, sphi, coh, ptc) && mc_plastic_step(m, st, sphi, spsi, coh, ptc, dps))
+            if (!mc_surely_elastic(m, st, sphi, coh, ptc) && mc_plastic_step<1>(m, st, sphi, spsi, coh, ptc, dps))
                 plasticStrain = plasticStrain + dps;
             /* in place, an unchanged value need not be stored */
             if (a.ps_out != a.ps || plasticStrain != a.ps[(size_t)t * E + e])
@@ -1384,18 +1622,6 @@ __device__ __forceinline__ double node_finish(const StepArgs& a, int n, double f
     a.xn[N + n] = x1 + dt * v1;
     a.xn[2 * N + n] = x2 + dt * v2;
     return vmag;
-}
-
-/* base[off / 8] for a uniform base and a per-lane byte offset below 4 GB (a
-   row of E or N doubles: device memory holds fewer than 2^29 elements): the
-   load takes its base from scalar registers and its offset from one vector
-   register, so a row costs no vector address arithmetic */
-typedef const __attribute__((address_space(1))) char* gbase;   /* uniform, in global memory */
-__device__ __forceinline__ gbase row_base(const double* p) { return (gbase)(uintptr_t)p; }
-__device__ __forceinline__ double ld_row(gbase base, size_t row, uint32_t off) {
-    gbase b = base + 8 * row;
-    asm("" : "+s"(b), "+v"(off));   /* keeps the row's base scalar and the offset 32 bits wide */
-    return *(const __attribute__((address_space(1))) double*)(b + off);
 }
 
 /* --------------------------------------------------------------------------
@@ -2796,11 +3022,12 @@ __device__ __forceinline__ int batch_member(const BatchGrid& g, int& b) {
 }
 
 template <int RSET, bool TW, bool MM>
-__global__ void __launch_bounds__(TW ? 640 : 64) k_elem_batch(BatchGrid g) {
+__global__ void __launch_bounds__(TW ? 64 * tw_waves(RSET) : 64, TW ? tw_occupancy(RSET) : 1) k_elem_batch(BatchGrid g) {
     int b;
     const int m = batch_member(g, b);
     if (b >= g.count[m]) return;
-    elem_pass<RSET, TW, MM>(member_args(g.base, g.mem, m), b, g.count[m]);
+    if constexpr (TW) elem_pass_tw<RSET, MM>(member_args(g.base, g.mem, m), b, g.count[m]);
+    else elem_pass<RSET, MM>(member_args(g.base, g.mem, m), b, g.count[m]);
 }
 
 template <int RSET, bool TW>
@@ -3058,6 +3285,8 @@ static void fill_dev_material(const snh_material& s, DevMaterial& d) {
     d.tanphi = tan(s.frictionAngle[0] * degrad);
     d.anphi0 = (1.0 + d.sphi) / (1.0 - d.sphi);
     d.sqanphi0 = sqrt(d.anphi0);
+    d.anpsi0 = (1.0 + d.spsi) / (1.0 - d.spsi);
+    d.rtanphi0 = d.tanphi > 0.0 ? 1.0 / d.tanphi : 0.0;
     d.vis_min = s.vis_min;
     d.vis_max = s.vis_max;
     d.refvisc = s.refvisc;
@@ -3160,6 +3389,19 @@ static void free_all(snh_context* c) {
                     c->topo_pfirst, c->rec_code};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+}
+
+/* The element-pass layout of a context that is not autotuned.  Tet per wave
+   fills its loads, tet per lane starts more and smaller blocks and lets fewer
+   tets wait for one that yields.  Measured (us, tet per lane / per wave):
+   elastic 9.5 / 10.7 at 8112 elements, 14.2 / 12.0 at 16384, 52 / 38 at
+   127000; Maxwell 11.1 / 12.9, 16.5 / 14.2, 65 / 50; Mohr-Coulomb extension
+   98 / 102 at 256000, 177 / 179 at 441000, 397 / 364 at 885000, and yielding
+   throughout 106 / 136, 199 / 236, 430 / 424; visco-plastic 111 / 117,
+   197 / 209, 473 / 429. */
+static int32_t default_elem_variant(int rset, int E) {
+    const bool soft = (rset & (RS_PLASTIC | RS_VISCOPLASTIC)) != 0;
+    return E >= (soft ? 700000 : 12000) ? SNH_ELEM_TET_PER_WAVE : SNH_ELEM_TET_PER_LANE;
 }
 
 extern "C" int snh_context_create(const snh_config* cfg, snh_context** out) {
@@ -3382,7 +3624,7 @@ extern "C" int snh_context_create(const snh_config* cfg, snh_context** out) {
         return rc;
     }
     c->cur = 0;
-    c->elem_variant = SNH_ELEM_TET_PER_LANE;
+    c->elem_variant = default_elem_variant(c->rset, c->E);
     c->node_band = 8;
     c->node_variant = SNH_NODE_PER_NODE;
     if (const char* nv = getenv("SNH_NODE_VARIANT")) c->node_variant = atoi(nv) == SNH_NODE_TILED ? SNH_NODE_TILED : SNH_NODE_PER_NODE;
@@ -3653,10 +3895,10 @@ static int launch_elem_fp64(snh_context* c, StepArgs a) {
         HIPCHK(hipGetLastError());
         return SNH_OK;
     }
-    const bool tw = c->elem_variant == SNH_ELEM_TET_PER_WAVE;
+    const bool tw = c->elem_variant == SNH_ELEM_TET_PER_WAVE || c->E > LANE_MOST_ELEMENTS;
     if (tw) {
         grid = dim3((c->E + 63) / 64);
-        block = dim3(640);
+        block = dim3(64 * tw_waves(c->rset));
     }
 #define TL_LAUNCH(R)                                                                          \
     do {                                                                                      \
@@ -4917,7 +5159,8 @@ static int ens_batch_step(const snh_ensemble* e, const EnsGroup& grp, hipStream_
         g[k] = BatchGrid{grp.base[p], grp.dmem[p], grp.dfirst[k], grp.dcount[k], grp.dmember[k]};
     }
     const dim3 ge(grp.grid[EB_ELEM]), gn(grp.grid[EB_NODE]), gg(grp.grid[EB_GEO]);
-    const dim3 be(e->tw ? 640 : 64);
+    const bool mx = c0->cfg.precision == SNH_PRECISION_MIXED;
+    const dim3 be(e->tw ? (mx ? 640 : 64 * tw_waves(c0->rset)) : 64);
     const bool tw = e->tw;
     if (c0->cfg.precision == SNH_PRECISION_MIXED) {
 #define EB_MX_LAUNCH(R)                                                                          \

@@ -57,8 +57,9 @@ struct DevMaterial {
     double tgf[8], tgd[8], tgc[8];
     double ten_off;
     double sphi, spsi, tanphi;  /* host libm sin/sin/tan of fa[0], da[0] */
-    double anphi0, sqanphi0;    /* (1 + sphi) / (1 - sphi) and its root, for the
-                                   elastic bound only */
+    double anphi0, sqanphi0;    /* (1 + sphi) / (1 - sphi) and its root */
+    double anpsi0;              /* (1 + spsi) / (1 - spsi) */
+    double rtanphi0;            /* 1 / tanphi, for the elastic bound only */
     /* viscosity */
     double vis_min, vis_max, refvisc, refsrate, reftemp, activationE, srexponent;
     int linear_visc;         /* srexponent == 1 and activationE == 0 */

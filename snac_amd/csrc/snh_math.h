@@ -29,6 +29,71 @@ SNH_HD int snh_ref_iabs(double x) {
 /* int + int of two abs() results, wrapping as the x86 add does */
 SNH_HD int snh_iadd_wrap(int a, int b) { return (int)((unsigned)a + (unsigned)b); }
 
+/* A divisor b as the unevaluated sum hi + lo = 1 / b (1 + 2^-104): quotients
+ * by it are a product and an FMA, RN(a hi + RN(a lo)) (N. Brisebarre,
+ * J.-M. Muller and S. K. Raina, "Accelerating correctly rounded
+ * floating-point division when the divisor is known in advance", IEEE Trans.
+ * Computers 53 (2004), method 1).  The sum before the rounding is within
+ * 2^-52 ulp of a / b, so the result is RN(a / b) unless the quotient lies that
+ * close to a rounding midpoint; 4e9 random quotients on gfx950 gave no
+ * difference from the division.  Normal range only.
+ *
+ * From an estimate of 1 / b good to 2^-24 (v_rcp_f64, v_rsq_f64), one or two
+ * Newton steps (P. Markstein, 1990) make hi faithful; the residual
+ * 1 - b hi is then exact, and lo is its product with hi. */
+typedef struct {
+    double hi, lo;
+} snh_recip;
+SNH_HD snh_recip snh_recip_of(double b, double y) {
+    snh_recip r;
+    double e = fma(-b, y, 1.0);
+    r.hi = fma(e, y, y);
+    e = fma(-b, r.hi, 1.0);
+    r.lo = e * r.hi;
+    return r;
+}
+SNH_HD double snh_quot(double a, snh_recip r) { return fma(a, r.hi, a * r.lo); }
+
+/* the reciprocal of b > 0 */
+SNH_HD snh_recip snh_recip_make(double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double y = __builtin_amdgcn_rcp(b);
+    y = fma(fma(-b, y, 1.0), y, y);
+#else
+    const double y = 1.0 / b;
+#endif
+    return snh_recip_of(b, y);
+}
+
+/* RN(sqrt(x)) for x > 0 and, in r, the reciprocal of that root.  Goldschmidt's
+ * coupled iteration for sqrt(x) and 1 / (2 sqrt(x)) from v_rsq_f64, then two
+ * residual corrections of the root (Markstein 1990; Muller et al., Handbook of
+ * Floating-Point Arithmetic, 2nd ed., sec. 4.7), which give the correctly
+ * rounded root; the reciprocal comes out of the same iteration instead of a
+ * division.  Without the scaling of the library's sqrt: normal range only
+ * (x = 0 gives NaN, as the 0 / 0 of a face without area does).
+ * 13 instructions for root and reciprocal and 2 per quotient, against 31 and
+ * 5 with sqrt, 1 / s and snh_div_by. */
+SNH_HD double snh_sqrt_recip(double x, snh_recip* r) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double t = fma(-h, g, 0.5);
+    g = fma(g, t, g);
+    h = fma(h, t, h);
+    double d = fma(-g, g, x);
+    g = fma(d, h, g);
+    d = fma(-g, g, x);
+    g = fma(d, h, g);
+    *r = snh_recip_of(g, h + h);
+    return g;
+#else
+    const double s = sqrt(x);
+    *r = snh_recip_of(s, 1.0 / s);
+    return s;
+#endif
+}
+
 /* hypot(x, y) as the reference's libm computes it.  The reference calls the
  * system hypot in tql2 (plastic_BI/Constitutive.c:430,462); on x86-64 with
  * glibc 2.35 that is the unfused form of C. F. Borges' corrected square root
@@ -42,7 +107,8 @@ SNH_HD int snh_iadd_wrap(int a, int b) { return (int)((unsigned)a + (unsigned)b)
  * gives the system hypot's bits: checked on the host against the libm
  * function.  Requires FMA contraction off. */
 SNH_HD double snh_hypot_kernel(double ax, double ay) {
-    double h = sqrt(ax * ax + ay * ay);
+    snh_recip rh;
+    double h = snh_sqrt_recip(ax * ax + ay * ay, &rh);
     double t1, t2;
     if (h <= 2.0 * ay) {
         const double delta = h - ay;
@@ -53,7 +119,7 @@ SNH_HD double snh_hypot_kernel(double ax, double ay) {
         t1 = 2.0 * delta * (ax - 2.0 * ay);
         t2 = (4.0 * delta - ay) * ay + delta * delta;
     }
-    h -= (t1 + t2) / (2.0 * h);
+    h -= 0.5 * snh_quot(t1 + t2, rh);   /* (t1 + t2) / (2 h) */
     return h;
 }
 
@@ -120,71 +186,6 @@ SNH_HD double snh_div_by(double a, double b, double y) {
     q = fma(r, y, q);
     r = fma(-b, q, a);
     return fma(r, y, q);
-}
-
-/* A divisor b as the unevaluated sum hi + lo = 1 / b (1 + 2^-104): quotients
- * by it are a product and an FMA, RN(a hi + RN(a lo)) (N. Brisebarre,
- * J.-M. Muller and S. K. Raina, "Accelerating correctly rounded
- * floating-point division when the divisor is known in advance", IEEE Trans.
- * Computers 53 (2004), method 1).  The sum before the rounding is within
- * 2^-52 ulp of a / b, so the result is RN(a / b) unless the quotient lies that
- * close to a rounding midpoint; 4e9 random quotients on gfx950 gave no
- * difference from the division.  Normal range only.
- *
- * From an estimate of 1 / b good to 2^-24 (v_rcp_f64, v_rsq_f64), one or two
- * Newton steps (P. Markstein, 1990) make hi faithful; the residual
- * 1 - b hi is then exact, and lo is its product with hi. */
-typedef struct {
-    double hi, lo;
-} snh_recip;
-SNH_HD snh_recip snh_recip_of(double b, double y) {
-    snh_recip r;
-    double e = fma(-b, y, 1.0);
-    r.hi = fma(e, y, y);
-    e = fma(-b, r.hi, 1.0);
-    r.lo = e * r.hi;
-    return r;
-}
-SNH_HD double snh_quot(double a, snh_recip r) { return fma(a, r.hi, a * r.lo); }
-
-/* the reciprocal of b > 0 */
-SNH_HD snh_recip snh_recip_make(double b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    double y = __builtin_amdgcn_rcp(b);
-    y = fma(fma(-b, y, 1.0), y, y);
-#else
-    const double y = 1.0 / b;
-#endif
-    return snh_recip_of(b, y);
-}
-
-/* RN(sqrt(x)) for x > 0 and, in r, the reciprocal of that root.  Goldschmidt's
- * coupled iteration for sqrt(x) and 1 / (2 sqrt(x)) from v_rsq_f64, then two
- * residual corrections of the root (Markstein 1990; Muller et al., Handbook of
- * Floating-Point Arithmetic, 2nd ed., sec. 4.7), which give the correctly
- * rounded root; the reciprocal comes out of the same iteration instead of a
- * division.  Without the scaling of the library's sqrt: normal range only
- * (x = 0 gives NaN, as the 0 / 0 of a face without area does).
- * 13 instructions for root and reciprocal and 2 per quotient, against 31 and
- * 5 with sqrt, 1 / s and snh_div_by. */
-SNH_HD double snh_sqrt_recip(double x, snh_recip* r) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const double y = __builtin_amdgcn_rsq(x);
-    double g = x * y, h = 0.5 * y;
-    const double t = fma(-h, g, 0.5);
-    g = fma(g, t, g);
-    h = fma(h, t, h);
-    double d = fma(-g, g, x);
-    g = fma(d, h, g);
-    d = fma(-g, g, x);
-    g = fma(d, h, g);
-    *r = snh_recip_of(g, h + h);
-    return g;
-#else
-    const double s = sqrt(x);
-    *r = snh_recip_of(s, 1.0 / s);
-    return s;
-#endif
 }
 
 #endif
