@@ -2793,6 +2793,29 @@ __global__ void __launch_bounds__(NODE_BLOCK) k_heat_node(StepArgs a) {
 /* --------------------------------------------------------------------------
  * k_geo: Snac_EP_LoopElementsMomentum's geometry and minLengthScale
  * ------------------------------------------------------------------------ */
+/* the least V / A over the faces of a tet (F_1EP27 without a face of any
+   area).  sqrt, halving and the division are monotone, so the face with the
+   largest sum of squares gives it exactly. */
+__device__ __forceinline__ double tet_min_length(const double X[4][3]) {
+    double ssq_max = 0.0, a0 = 0, b0 = 0, c0 = 0;
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+        double fa, fb, fc;
+        face_cross(X[kFaceToNode[f][0]], X[kFaceToNode[f][1]], X[kFaceToNode[f][2]], fa, fb, fc);
+        if (f == 0) {
+            a0 = fa;
+            b0 = fb;
+            c0 = fc;
+        }
+        double ssq = fa * fa + fb * fb + fc * fc;
+        ssq_max = ssq > ssq_max ? ssq : ssq_max;
+    }
+    const double V = tet_volume_from_face0(X[0], X[3], a0, b0, c0);
+    snh_recip rs;
+    (void)snh_sqrt_recip(ssq_max, &rs);
+    return ssq_max > 0.0 ? 2.0 * snh_quot(V, rs) : F_1EP27;   /* V / (sqrt / 2) */
+}
+
 __device__ __forceinline__ void geo_pass(StepArgs a, const int blk, const int nblk) {
     __shared__ double sh[GEO_BLOCK / 64];
     const int e = xcd_block(blk, nblk) * blockDim.x + threadIdx.x;
@@ -2810,28 +2833,8 @@ __device__ __forceinline__ void geo_pass(StepArgs a, const int blk, const int nb
             for (int q = 0; q < 4; q++)
 #pragma unroll
                 for (int d = 0; d < 3; d++) Xt[q][d] = X[kTetraToNode[t][q]][d];
-            /* min over faces of V / (sqrt(ssq)/2): sqrt, halving and the
-               division are monotone, so the face with the largest sum of
-               squares gives the minimum exactly */
-            double ssq_max = 0.0, a0 = 0, b0 = 0, c0 = 0;
-#pragma unroll
-            for (int f = 0; f < 4; f++) {
-                double fa, fb, fc;
-                face_cross(Xt[kFaceToNode[f][0]], Xt[kFaceToNode[f][1]], Xt[kFaceToNode[f][2]], fa, fb, fc);
-                if (f == 0) {
-                    a0 = fa;
-                    b0 = fb;
-                    c0 = fc;
-                }
-                double ssq = fa * fa + fb * fb + fc * fc;
-                ssq_max = ssq > ssq_max ? ssq : ssq_max;
-            }
-            const double V = tet_volume_from_face0(Xt[0], Xt[3], a0, b0, c0);
-            const double area = sqrt(ssq_max) / 2.0;
-            if (area) {
-                double ls = fabs(V / area);
-                if (emin > ls) emin = ls;
-            }
+            const double ls = tet_min_length(Xt);
+            if (emin > ls) emin = ls;
         }
     }
     double bm = block_min(emin, sh);
@@ -2841,13 +2844,54 @@ __device__ __forceinline__ void geo_pass(StepArgs a, const int blk, const int nb
     }
 }
 
+/* The same with five waves to 64 elements, wave w taking tets w and w + 5: on
+   a mesh with fewer elements than the GPU has lanes a tet then waits for one
+   other and not for nine. A step of the elastic box, tets in one lane / over
+   five waves: 22.2 / 20.9 us at 16 x 8 x 16 (2048 elements), 29.9 / 28.8 at
+   16384, 49.3 / 50.2 at 55296, 146 / 150 at 255905: every corner is read by
+   five waves instead of one. */
+#define GEO_TETS_BLOCK 320
+#define GEO_TETS_MOST 20000
+__device__ __forceinline__ void geo_pass_tets(StepArgs a, const int blk, const int nblk) {
+    __shared__ double sh[GEO_TETS_BLOCK / 64];
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int e = xcd_block(blk, nblk) * 64 + (int)(threadIdx.x & 63);
+    double emin = INFINITY;
+    if (e < a.E) {
+        const int eq = (int)fastdiv((uint32_t)e, a.dEI);
+        /* the element's lowest node (elem_pass_tw) */
+        const uint32_t no = 8u * (uint32_t)(e + eq + a.I * (int)fastdiv((uint32_t)eq, a.dEJ));
+        emin = F_1EP27;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            double X[4][3];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int h = tet_node(w + 5 * u, q);
+                const size_t c = (size_t)(((h ^ (h >> 1)) & 1) + a.I * (((h >> 1) & 1) + a.J * (h >> 2)));
+#pragma unroll
+                for (int d = 0; d < 3; d++) X[q][d] = ld_row(row_base(a.xc), c + (size_t)d * (size_t)a.N, no);
+            }
+            const double ls = tet_min_length(X);
+            if (emin > ls) emin = ls;
+        }
+    }
+    const double bm = block_min(emin, sh);
+    if (threadIdx.x == 0) {
+        a.part_min[blk] = bm;
+        if (blk == 0) a.scal->dt_rot = a.scal->dt;
+    }
+}
+__global__ void __launch_bounds__(GEO_TETS_BLOCK) k_geo_tets(StepArgs a) {
+    geo_pass_tets(a, (int)blockIdx.x, (int)gridDim.x);
+}
+
 __global__ void __launch_bounds__(GEO_BLOCK) k_geo(StepArgs a) { geo_pass(a, (int)blockIdx.x, (int)gridDim.x); }
 
 /* --------------------------------------------------------------------------
  * k_fin: _Snac_Context_Sync
  * ------------------------------------------------------------------------ */
-__device__ __forceinline__ void fin_pass(StepArgs a, const int nmin, const int nvmax) {
-    __shared__ double sh[FIN_BLOCK / 64];
+__device__ __forceinline__ void fin_pass(StepArgs a, const int nmin, const int nvmax, double* sh) {
     double mn = INFINITY, mx = -INFINITY;
     /* eight partials in flight per thread: indices past the end read the
        last partial again, which leaves a minimum or maximum unchanged (and
@@ -2887,7 +2931,10 @@ __device__ __forceinline__ void fin_pass(StepArgs a, const int nmin, const int n
     }
 }
 
-__global__ void __launch_bounds__(FIN_BLOCK) k_fin(StepArgs a, int nmin, int nvmax) { fin_pass(a, nmin, nvmax); }
+__global__ void __launch_bounds__(FIN_BLOCK) k_fin(StepArgs a, int nmin, int nvmax) {
+    __shared__ double sh[FIN_BLOCK / 64];
+    fin_pass(a, nmin, nvmax, sh);
+}
 
 /* --------------------------------------------------------------------------
  * Batched launches of an ensemble: one grid over the blocks of several
@@ -3065,8 +3112,9 @@ __global__ void __launch_bounds__(GEO_BLOCK) k_geo_batch(BatchGrid g) {
 __global__ void __launch_bounds__(FIN_BLOCK) k_fin_batch(StepArgs base, const BatchMember* __restrict__ mem,
                                                          const int* __restrict__ nmin,
                                                          const int* __restrict__ nvmax) {
+    __shared__ double sh[FIN_BLOCK / 64];
     const int m = (int)blockIdx.x;
-    fin_pass(member_args(base, mem, m), nmin[m], nvmax[m]);
+    fin_pass(member_args(base, mem, m), nmin[m], nvmax[m], sh);
 }
 
 /* minLengthScale after a remesh: the running minimum of
@@ -3153,6 +3201,7 @@ struct snh_context {
     int topo_threads;   /* sweep block: a power of two >= min(I, K) */
     int n_geo_blocks, n_node_blocks;
     int n_slot_blocks;  /* blocks of the slot-per-wave node gather */
+    int n_min_parts;    /* block minima of V / A written by the last geometry pass */
     unsigned rset;  /* rheologies present */
     bool zero_done;
     bool rotation_pending;
@@ -3503,7 +3552,7 @@ extern "C" int snh_context_create(const snh_config* cfg, snh_context** out) {
     if (c->needs_plastic) ALLOC(c->ps, 10 * E * sizeof(double));
     if (c->needs_visc) ALLOC(c->visc, 10 * E * sizeof(double));
     ALLOC(c->bc, N);
-    ALLOC(c->part_min, (size_t)c->n_geo_blocks * sizeof(double));
+    ALLOC(c->part_min, ((E + 63) / 64) * sizeof(double));
     c->node_kc = 8;
     if (const char* kc = getenv("SNH_NODE_KC")) c->node_kc = atoi(kc) > 0 ? atoi(kc) : 8;
     c->n_tile_blocks = ((c->I + NT_I - 1) / NT_I) * ((c->J + NT_J - 1) / NT_J) * ((c->K + c->node_kc - 1) / c->node_kc);
@@ -3789,10 +3838,19 @@ extern "C" int snh_upload_state(snh_context* c, const snh_state* s) {
     return clear_firewalls(c);
 }
 
+/* the geometry pass on the mesh of a, and how many block minima it leaves */
+static void launch_geo_args(snh_context* c, const StepArgs& a) {
+    if (c->E <= GEO_TETS_MOST) {
+        c->n_min_parts = (c->E + 63) / 64;
+        hipLaunchKernelGGL(k_geo_tets, dim3(c->n_min_parts), dim3(GEO_TETS_BLOCK), 0, c->stream, a);
+    } else {
+        c->n_min_parts = c->n_geo_blocks;
+        hipLaunchKernelGGL(k_geo, dim3(c->n_geo_blocks), dim3(GEO_BLOCK), 0, c->stream, a);
+    }
+}
 static int launch_geo(snh_context* c) {
     KTimer kt(c, KK_GEO);
-    StepArgs a = make_args(c);
-    hipLaunchKernelGGL(k_geo, dim3(c->n_geo_blocks), dim3(GEO_BLOCK), 0, c->stream, a);
+    launch_geo_args(c, make_args(c));
     HIPCHK(hipGetLastError());
     return SNH_OK;
 }
@@ -3800,7 +3858,7 @@ static int launch_geo(snh_context* c) {
 static int launch_fin(snh_context* c) {
     KTimer kt(c, KK_FIN);
     StepArgs a = make_args(c);
-    hipLaunchKernelGGL(k_fin, dim3(1), dim3(FIN_BLOCK), 0, c->stream, a, c->n_geo_blocks, c->n_vmax_parts);
+    hipLaunchKernelGGL(k_fin, dim3(1), dim3(FIN_BLOCK), 0, c->stream, a, c->n_min_parts, c->n_vmax_parts);
     HIPCHK(hipGetLastError());
     return SNH_OK;
 }
@@ -4136,7 +4194,7 @@ extern "C" int snh_remesh(snh_context* c, const snh_state* s) {
        running minimum of the length scale */
     if ((rc = launch_geo(c))) return rc;
     StepArgs a = make_args(c);
-    hipLaunchKernelGGL(k_minlen_merge, dim3(1), dim3(FIN_BLOCK), 0, c->stream, a, c->n_geo_blocks);
+    hipLaunchKernelGGL(k_minlen_merge, dim3(1), dim3(FIN_BLOCK), 0, c->stream, a, c->n_min_parts);
     HIPCHK(hipGetLastError());
     c->rotation_pending = true;
     HIPCHK(hipStreamSynchronize(c->stream));

@@ -219,8 +219,8 @@ static int adj_run_tape(snh_context* c, AdjointCtx* A, uint32_t t0, int i0, int 
         launch_node_fp64(c, an);
         StepArgs ag = a;
         ag.xc = a.xn;
-        hipLaunchKernelGGL(k_geo, dim3(c->n_geo_blocks), dim3(GEO_BLOCK), 0, c->stream, ag);
-        hipLaunchKernelGGL(k_fin, dim3(1), dim3(FIN_BLOCK), 0, c->stream, ag, c->n_geo_blocks, c->n_vmax_parts);
+        launch_geo_args(c, ag);
+        hipLaunchKernelGGL(k_fin, dim3(1), dim3(FIN_BLOCK), 0, c->stream, ag, c->n_min_parts, c->n_vmax_parts);
         if (hipGetLastError() != hipSuccess) rc = set_err(SNH_EHIP, "adjoint tape step launch failed");
     }
     return rc;
