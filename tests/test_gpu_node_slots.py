@@ -36,3 +36,11 @@ def test_other_dt_types(dt_type):
     p = P.elastic_box_compression(elements=(64, 3, 5), extent_km=(128.0, 6.0, 10.0))
     p.dtType, p.timeStep = dt_type, 1.0e-3
     _same(p, 6)
+
+
+# above 400000 nodes the per-node gather, whose rows are turned within bands
+# of 16 planes: fewer rows than the turn, a last band of one, three and sixteen
+# planes, rows shorter than a block
+@pytest.mark.parametrize("elements", [(750, 1, 272), (1200, 2, 114), (30, 25, 511)], ids=str)
+def test_turned_rows(elements):
+    _same(P.elastic_box_compression(elements=elements, extent_km=tuple(2.0 * e for e in elements)), 2)
