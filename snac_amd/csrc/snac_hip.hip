@@ -2291,17 +2291,20 @@ __global__ void __launch_bounds__(NT_THREADS) k_node_tile(StepArgs a) {
  *
  * k_topo_prep (one thread per top node) computes everything the sweep does
  * not change -- the node's gradient for the running maximum, the
- * differences with its old +x/+z neighbours and the stencil's denominators
- * with their correctly rounded reciprocals -- into records stored in
+ * differences with its old +x/+z neighbours and the reciprocals of the
+ * stencil's denominators as pairs hi + lo -- into records stored in
  * diagonal order, and reduces the maximum and the first node (in node
  * order) whose gradient reaches the criterion per block.  k_topo (one
  * block) finishes the reductions and sweeps the diagonals with the heights
  * of diagonal d-1 in LDS, prefetching records several diagonals ahead
- * (written by k_topo_prep on all XCDs just before); a
- * division whose divisor the sweep does not change is done as
- * snh_div_by with the stored reciprocal (correctly rounded, as the
- * reference's).  Both run after k_node with its arguments: xc the old
- * coordinates, xn the updated ones, whose heights k_topo finalises.
+ * (written by k_topo_prep on all XCDs just before).  A diagonal is bound by
+ * its chain of dependent FP64 operations, the LDS hand-over and the issue of
+ * one wave's instructions: a division is snh_quot with the stored pair (two
+ * operations for five with divisor and reciprocal), and a record six loads
+ * from scalar bases for eleven.  193 diagonals of a 128 x 66 surface: 86.6 us
+ * with single fields, divisors and reciprocals, 64.3 us so.  Both run after
+ * k_node with its arguments: xc the old coordinates, xn the updated ones,
+ * whose heights k_topo finalises.
  * ------------------------------------------------------------------------ */
 #define TOPO_REC 11          /* doubles per top-node record            */
 #define TOPO_PREP_BLOCK 256
@@ -2337,6 +2340,19 @@ __host__ __device__ __forceinline__ long long topo_off(int d, int I, int K) {
     return a - b;
 }
 
+/* a divisor as the pair that snh_quot takes, and back */
+__device__ __forceinline__ void topo_divisor(double b, double* r) {
+    const snh_recip q = snh_recip_of(b, 1.0 / b);
+    r[0] = q.hi;
+    r[1] = q.lo;
+}
+__device__ __forceinline__ double topo_quot(double x, const double* r) {
+    snh_recip q;
+    q.hi = r[0];
+    q.lo = r[1];
+    return snh_quot(x, q);
+}
+
 __global__ void __launch_bounds__(TOPO_PREP_BLOCK) k_topo_prep(StepArgs a, TopoArgs t) {
     __shared__ double smax[TOPO_PREP_BLOCK];
     __shared__ int sfirst[TOPO_PREP_BLOCK];
@@ -2365,20 +2381,16 @@ __global__ void __launch_bounds__(TOPO_PREP_BLOCK) k_topo_prep(StepArgs a, TopoA
                 const double xR = a.xc[n + 1], yR = a.xc[N + n + 1];
                 dydx1 = (yR - y0) / (xR - x0);
                 r[1] = dydx1;
-                r[2] = x0 - xL;
-                r[3] = 1.0 / r[2];
-                r[4] = 0.5 * (xR - xL);
-                r[5] = 1.0 / r[4];
+                topo_divisor(x0 - xL, &r[2]);
+                topo_divisor(0.5 * (xR - xL), &r[4]);
             }
             if (alz) {
                 const double z0 = a.xn[2 * N + n], zB = a.xn[2 * N + n - IJ];
                 const double yF = a.xc[N + n + IJ], zF = a.xc[2 * N + n + IJ];
                 dydz1 = (yF - y0) / (zF - z0);
                 r[6] = dydz1;
-                r[7] = z0 - zB;
-                r[8] = 1.0 / r[7];
-                r[9] = 0.5 * (zF - zB);
-                r[10] = 1.0 / r[9];
+                topo_divisor(z0 - zB, &r[7]);
+                topo_divisor(0.5 * (zF - zB), &r[9]);
             }
             /* getMaxTopoGrad's dydx, dydz are the same quotients */
             g = (alx && alz) ? sqrt(dydx1 * dydx1 + dydz1 * dydz1)
@@ -2389,8 +2401,13 @@ __global__ void __launch_bounds__(TOPO_PREP_BLOCK) k_topo_prep(StepArgs a, TopoA
             if (alz && k == 0) r[6] = a.xc[N + n + IJ];   /* old height of (i, 1)  */
         }
         if (t.mode == TOPO_SURFACE) {
-#pragma unroll
-            for (int q = 0; q < TOPO_REC; q++) t.rec[q * PP + pos] = r[q];
+            double2* const o = (double2*)t.rec + pos;
+            o[0] = make_double2(r[0], r[1]);
+            o[PP] = make_double2(r[2], r[3]);
+            o[2 * PP] = make_double2(r[4], r[5]);
+            o[3 * PP] = make_double2(r[7], r[8]);
+            o[4 * PP] = make_double2(r[9], r[10]);
+            t.rec[10 * PP + pos] = r[6];
         } else {
             /* one line per row (along x) or column (along z): the height and
                the direction's five fields, 64 bytes per node in line order */
@@ -2449,6 +2466,22 @@ __device__ int topo_reduce(const StepArgs& a, const TopoArgs& t, double* rmax, i
     return pfirst;
 }
 
+/* the record at position at + off of the surface's P, fields as k_topo_prep
+   numbers them: five rows of pairs and one of the field 6, each read from a
+   scalar base */
+__device__ __forceinline__ void topo_record(const double* rec, size_t P, int at, uint32_t off, double r[TOPO_REC]) {
+    typedef double pair __attribute__((ext_vector_type(2)));
+    constexpr int field[5] = {0, 2, 4, 7, 9};
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+        const gbase b = row_base(rec) + 16 * (q * P + (size_t)at);
+        const pair v = *(const __attribute__((address_space(1))) pair*)(b + 16u * off);
+        r[field[q]] = v.x;
+        r[field[q] + 1] = v.y;
+    }
+    r[6] = *(const __attribute__((address_space(1))) double*)(row_base(rec) + 8 * (10 * P + (size_t)at) + 8u * off);
+}
+
 /* BLOCK: the most threads the sweep may be launched with (a diagonal's
    nodes, at most min(I, K)); PF: diagonals prefetched ahead -- deeper with
    the smaller block, whose waves may hold more registers */
@@ -2474,14 +2507,18 @@ __global__ void __launch_bounds__(BLOCK) k_topo(StepArgs a, TopoArgs t) {
        loads before their use three barriers later. */
     const int D = I + K - 1;
     double ring[TOPO_PF][TOPO_REC];
+    int at = 0, dn = 0, ilo_n = 0;   /* diagonal to load next: its first record and first i */
+    auto next_records = [&](double* r) {
+        const int cn = min(dn, I - 1) - ilo_n + 1;
+        topo_record(t.rec, PP, at, (uint32_t)min(tid, cn - 1), r);
+        if (dn < D - 1) {
+            dn++;
+            at += cn;
+            ilo_n = topo_ilo(dn, K);
+        }
+    };
 #pragma unroll
-    for (int r = 0; r < TOPO_PF; r++) {
-        const int dd = r < D ? r : D - 1;
-        const int cn = (dd < I - 1 ? dd : I - 1) - topo_ilo(dd, K) + 1;
-        const size_t pos = (size_t)topo_off(dd, I, K) + (tid < cn ? tid : cn - 1);
-#pragma unroll
-        for (int q = 0; q < TOPO_REC; q++) ring[r][q] = t.rec[q * PP + pos];
-    }
+    for (int r = 0; r < TOPO_PF; r++) next_records(ring[r]);
     for (int d0 = 0; d0 < D; d0 += TOPO_PF) {
 #pragma unroll
         for (int r = 0; r < TOPO_PF; r++) {
@@ -2497,10 +2534,10 @@ __global__ void __launch_bounds__(BLOCK) k_topo(StepArgs a, TopoArgs t) {
             const double* rc = ring[r];
             const double y0 = rc[0];
             /* DiffTopo + UpdateInteriorTopo */
-            const double dydx2 = snh_div_by(y0 - yl, rc[2], rc[3]);
-            const double d2ydx2 = snh_div_by(rc[1] - dydx2, rc[4], rc[5]);
-            const double dydz2 = snh_div_by(y0 - yb, rc[7], rc[8]);
-            const double d2ydz2 = snh_div_by(rc[6] - dydz2, rc[9], rc[10]);
+            const double dydx2 = topo_quot(y0 - yl, rc + 2);
+            const double d2ydx2 = topo_quot(rc[1] - dydx2, rc + 4);
+            const double dydz2 = topo_quot(y0 - yb, rc + 7);
+            const double d2ydz2 = topo_quot(rc[6] - dydz2, rc + 9);
             const double lapl_topo = d2ydx2 + d2ydz2;
             const double yi = y0 + kd * lapl_topo;
             /* AdjustEdgeTopo: xN1 along x, xN2 along z, the old height of a
@@ -2513,13 +2550,7 @@ __global__ void __launch_bounds__(BLOCK) k_topo(StepArgs a, TopoArgs t) {
             const double y = active ? ((h1 || h2) ? ye : yi) : y0;
             if (valid) yd[d & 1][i] = y;
             if (active) a.xn[N + I * (J - 1) + i + IJ * k] = y;
-            {
-                const int dn = d + TOPO_PF < D ? d + TOPO_PF : D - 1;
-                const int cn = (dn < I - 1 ? dn : I - 1) - topo_ilo(dn, K) + 1;
-                const size_t pos = (size_t)topo_off(dn, I, K) + (tid < cn ? tid : cn - 1);
-#pragma unroll
-                for (int q = 0; q < TOPO_REC; q++) ring[r][q] = t.rec[q * PP + pos];
-            }
+            next_records(ring[r]);
             __syncthreads();
         }
     }
@@ -2567,8 +2598,8 @@ __global__ void __launch_bounds__(64) k_topo_line(StepArgs a, TopoArgs t) {
             const int s = s0 + r;
             const double* rc = ring[r];
             const double y0 = rc[0];
-            const double dy2 = snh_div_by(y0 - yl, rc[2], rc[3]);
-            const double lapl_topo = snh_div_by(rc[1] - dy2, rc[4], rc[5]);
+            const double dy2 = topo_quot(y0 - yl, rc + 2);
+            const double lapl_topo = topo_quot(rc[1] - dy2, rc + 4);
             const double yi = y0 + kd * lapl_topo;
             /* AdjustEdgeTopo: the first node copies the old height of its
                + neighbour, the last the final height of its - neighbour */

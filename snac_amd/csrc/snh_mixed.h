@@ -318,10 +318,10 @@ __device__ __forceinline__ void node_pass_mx(StepArgs a, const int blk, const in
     const int g = xcd_block(blk, nblk) * blockDim.x + threadIdx.x;
     double vmag = -INFINITY;
     if (g < a.N) {
-        /* the FP64 gather's banded node order: node rows that read one
-           element row run close together and share its L2 */
+        /* the FP64 gather's node order: 110 us at 130x35x97 elements, 113 in
+           bands without the turn */
         int i, j, k;
-        const int n = gather_node(a, g, i, j, k);
+        const int n = gather_node_turned(a, g, i, j, k);
         const double dt = a.scal->dt;
         const double c = a.scal->speedOfSound;
         const double rc2 = 1.0 / (c * c);
