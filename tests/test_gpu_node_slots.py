@@ -44,3 +44,13 @@ def test_other_dt_types(dt_type):
 @pytest.mark.parametrize("elements", [(750, 1, 272), (1200, 2, 114), (30, 25, 511)], ids=str)
 def test_turned_rows(elements):
     _same(P.elastic_box_compression(elements=elements, extent_km=tuple(2.0 * e for e in elements)), 2)
+
+
+# the heat gather in both forms: up to 200000 nodes and above; the stress holds
+# the temperature (density, viscosity) of the steps before
+@pytest.mark.parametrize("elements", [(5, 3, 9), (64, 3, 5), (62, 30, 99), (63, 31, 97)], ids=str)
+def test_heat(elements):
+    p = P.maxwell_thermal(elements=elements, extent_km=tuple(2.0 * e for e in elements))
+    ref, got, _, _ = run_both(p, 3)
+    for f in ("velocity", "stress"):
+        assert np.array_equal(ref[f], got[f]), f
