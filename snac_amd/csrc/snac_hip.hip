@@ -973,6 +973,7 @@ __device__ __forceinline__ void elem_pass(StepArgs a, const int blk, const int n
      Mohr-Coulomb and 1026 us visco-plastic, against 920 and 1075 us with five
      (their return diverges, and a wave then does it for both its tets) and
      1160 and 1445 us with ten waves held to 96 registers.
+   (The four take 658, 797, 860 and 1008 us with the later arithmetic.)
    What bounds it now is the wait for its loads and barriers: at 884 us the
    Mohr-Coulomb pass issues VALU instructions 35 % of the time and moves 2.4 GB
    at 2.7 TB/s. */
