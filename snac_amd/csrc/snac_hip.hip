@@ -4095,12 +4095,12 @@ static int launch_elem_fp64(snh_context* c, StepArgs a) {
         return SNH_OK;
     }
     const bool tw = c->elem_variant == SNH_ELEM_TET_PER_WAVE || c->E > LANE_MOST_ELEMENTS;
-    if (tw) {
-        grid = dim3((c->E + 63) / 64);
-        block = dim3(64 * tw_waves(c->rset));
-    }
+    if (tw) grid = dim3((c->E + 63) / 64);
+    /* the waves are those of the instantiation launched: a mix of laws takes
+       the kernel of all four, whatever is in the mix */
 #define TL_LAUNCH(R)                                                                          \
     do {                                                                                      \
+        block = dim3(tw ? 64 * tw_waves(R) : 64);                                             \
         if (mm) {                                                                             \
             if (tw) hipLaunchKernelGGL((k_elem<R, true, true>), grid, block, 0, c->stream, a); \
             else hipLaunchKernelGGL((k_elem<R, false, true>), grid, block, 0, c->stream, a);  \
@@ -5367,10 +5367,9 @@ static int ens_batch_step(const snh_ensemble* e, const EnsGroup& grp, hipStream_
         g[k] = BatchGrid{grp.base[p], grp.dmem[p], grp.dfirst[k], grp.dcount[k], grp.dmember[k]};
     }
     const dim3 ge(grp.grid[EB_ELEM]), gn(grp.grid[EB_NODE]), gg(grp.grid[EB_GEO]);
-    const bool mx = c0->cfg.precision == SNH_PRECISION_MIXED;
-    const dim3 be(e->tw ? (mx ? 640 : 64 * tw_waves(c0->rset)) : 64);
     const bool tw = e->tw;
     if (c0->cfg.precision == SNH_PRECISION_MIXED) {
+        const dim3 be(tw ? 640 : 64);
 #define EB_MX_LAUNCH(R)                                                                          \
     do {                                                                                         \
         if (tw) hipLaunchKernelGGL((k_elem_mx_batch<R, true>), ge, be, 0, s, g[EB_ELEM]);        \
@@ -5386,6 +5385,7 @@ static int ens_batch_step(const snh_ensemble* e, const EnsGroup& grp, hipStream_
     } else {
 #define EB_ELEM_LAUNCH(R)                                                                        \
     do {                                                                                         \
+        const dim3 be(tw ? 64 * tw_waves(R) : 64);                                               \
         if (mm) {                                                                                \
             if (tw) hipLaunchKernelGGL((k_elem_batch<R, true, true>), ge, be, 0, s, g[EB_ELEM]); \
             else hipLaunchKernelGGL((k_elem_batch<R, false, true>), ge, be, 0, s, g[EB_ELEM]);   \
