@@ -4840,6 +4840,7 @@ static int autotune_node(snh_context* c, snh_tune_report& rep) {
     ok = ok && hipEventCreate(&e0) == hipSuccess && hipEventCreate(&e1) == hipSuccess;
     int rc = ok ? SNH_OK : set_err(SNH_ENOMEM, "autotune scratch allocation failed");
     const int saved_v = c->node_variant, saved_kc = c->node_kc, saved_tb = c->n_tile_blocks;
+    const int saved_parts = c->n_vmax_parts;   /* of the context's own buffer */
     for (int o = 0; o < SNH_NODE_TUNES && rc == SNH_OK; o++) {
         c->node_variant = o == 0 ? SNH_NODE_PER_NODE : SNH_NODE_TILED;
         c->node_kc = o == 0 ? saved_kc : kcs[o - 1];
@@ -4865,6 +4866,7 @@ static int autotune_node(snh_context* c, snh_tune_report& rep) {
     c->node_variant = saved_v;
     c->node_kc = saved_kc;
     c->n_tile_blocks = saved_tb;
+    c->n_vmax_parts = saved_parts;
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
     void* p[] = {sv, sx, spv};
@@ -4881,6 +4883,7 @@ static int autotune_node(snh_context* c, snh_tune_report& rep) {
         double* pv = nullptr;
         HIPCHK(hipStreamSynchronize(c->stream));
         HIPCHK(hipMalloc((void**)&pv, (size_t)tb * sizeof(double)));
+        HIPCHK(ctx_copy(c, pv, c->part_vmax, (size_t)c->n_vmax_parts * sizeof(double), hipMemcpyDeviceToDevice));
         (void)hipFree(c->part_vmax);
         c->part_vmax = pv;
     }
@@ -5132,6 +5135,9 @@ struct EnsGroup {
 struct snh_ensemble {
     std::vector<snh_context*> m;
     std::vector<int> cur0;      /* members' coordinate-buffer index at capture */
+    /* block partials that a graph launch leaves in each member's buffers:
+       minima of V / A, maxima of |v| */
+    std::vector<int> min_parts, vmax_parts;
     int graph_steps;
     hipStream_t origin;
     hipEvent_t fork;
@@ -5241,6 +5247,11 @@ static int ens_make_groups(snh_ensemble* e) {
     return SNH_OK;
 }
 
+/* a member's blocks in the batched node pass */
+static int batch_node_blocks(const snh_context* c) {
+    return c->cfg.precision == SNH_PRECISION_MIXED ? c->n_node_blocks : c->n_slot_blocks;
+}
+
 /* device tables of a group's batched launches; its members' StepArgs for
    both coordinate-buffer parities, relative to its first member's */
 static int ens_batch_tables(snh_ensemble* e, EnsGroup& grp) {
@@ -5253,7 +5264,7 @@ static int ens_batch_tables(snh_ensemble* e, EnsGroup& grp) {
     for (int i = 0; i < n; i++) {
         const snh_context* c = e->m[grp.idx[i]];
         cnt[EB_ELEM][i] = (int)(e->tw ? (c->E + 63) / 64 : (c->E + EPW - 1) / EPW);
-        cnt[EB_NODE][i] = c->cfg.precision == SNH_PRECISION_MIXED ? c->n_node_blocks : c->n_slot_blocks;
+        cnt[EB_NODE][i] = batch_node_blocks(c);
         cnt[EB_GEO][i] = c->n_geo_blocks;
     }
     for (int k = 0; k < 3; k++) {
@@ -5445,6 +5456,14 @@ extern "C" int snh_ensemble_create(snh_context* const* members, int32_t n, int32
     e->join.assign(n, nullptr);
     e->cur0.resize(n);
     for (int i = 0; i < n; i++) e->cur0[i] = members[i]->cur;
+    /* what the members' buffers hold until a graph has run */
+    std::vector<int> min0(n), vmax0(n);
+    for (int i = 0; i < n; i++) {
+        min0[i] = members[i]->n_min_parts;
+        vmax0[i] = members[i]->n_vmax_parts;
+    }
+    e->min_parts.resize(n);
+    e->vmax_parts.resize(n);
     int rc = SNH_OK;
     do {
         if (hipStreamCreateWithFlags(&e->origin, hipStreamNonBlocking) != hipSuccess ||
@@ -5508,8 +5527,17 @@ extern "C" int snh_ensemble_create(snh_context* const* members, int32_t n, int32
             if (hipGraphInstantiate(&e->exec[par], g, nullptr, nullptr, 0) != hipSuccess)
                 rc = set_err(SNH_EHIP, "hipGraphInstantiate failed");
         }
-        for (int i = 0; i < n; i++) e->m[i]->cur = e->cur0[i];
+        for (int i = 0; i < n; i++) {
+            snh_context* c = e->m[i];
+            c->cur = e->cur0[i];
+            e->min_parts[i] = e->batched ? c->n_geo_blocks : c->n_min_parts;
+            e->vmax_parts[i] = e->batched ? batch_node_blocks(c) : c->n_vmax_parts;
+        }
     } while (0);
+    for (int i = 0; i < n; i++) {   /* the captured passes have not run */
+        members[i]->n_min_parts = min0[i];
+        members[i]->n_vmax_parts = vmax0[i];
+    }
     if (rc) {
         ens_free(e);
         return rc;
@@ -5535,9 +5563,12 @@ extern "C" int snh_ensemble_step(snh_ensemble* e, int32_t nsteps) {
         }
     for (int r = 0; r < reps; r++) {
         HIPCHK(hipGraphLaunch(e->exec[par], e->origin));
-        for (snh_context* c : e->m) {
+        for (size_t i = 0; i < e->m.size(); i++) {
+            snh_context* c = e->m[i];
             c->timeStep += e->graph_steps;
             c->rotation_pending = true;
+            c->n_min_parts = e->min_parts[i];
+            c->n_vmax_parts = e->vmax_parts[i];
         }
     }
     if (rest) {
