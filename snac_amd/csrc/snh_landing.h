@@ -72,6 +72,7 @@ class Landing {
     /* bytes from device memory src to dst, after what the stream holds; src
        may be overwritten by later work of the same stream */
     hipError_t push(void* dst, const void* src, size_t bytes) {
+        pushed_ = true;
         if (!open_) {
             hipError_t r = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream_);
             return r != hipSuccess ? r : hipStreamSynchronize(stream_);
@@ -98,9 +99,11 @@ class Landing {
         }
         return hipSuccess;
     }
-    /* every pushed byte is in its place */
+    /* every pushed byte is in its place, and the stream's work is done also
+       when there was none to push */
     hipError_t finish() {
         close();
+        if (!pushed_) return hipStreamSynchronize(stream_);
         return hipError_t(error_.load());
     }
 
@@ -190,7 +193,7 @@ class Landing {
     }
 
     hipStream_t stream_;
-    bool open_ = false, closed_ = false, done_ = false;
+    bool open_ = false, pushed_ = false, closed_ = false, done_ = false;
     int slots_ = 0, index_[LAND_SLOTS] = {};
     void* slot_[LAND_SLOTS] = {};
     Job job_[LAND_SLOTS];
