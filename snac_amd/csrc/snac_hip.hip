@@ -4955,12 +4955,8 @@ extern "C" int snh_autotune(snh_context* c, snh_tune_report* out) {
         return rc;
     }
     int best = 0;
-    /* tet per lane unless another is 10 % faster: beside other contexts' work
-       its many small blocks do better than alone (twelve yielding models of
-       12000-96000 elements: 91 ms for 200 steps, against 110 ms with the
-       layouts that were up to 10 % faster alone) */
     for (int v = 1; v < SNH_ELEM_VARIANTS; v++)
-        if (rep.elem_ms[v] < (best ? rep.elem_ms[best] : 0.9f * rep.elem_ms[0])) best = v;
+        if (rep.elem_ms[v] < rep.elem_ms[best]) best = v;
     c->elem_variant = best;
     if (getenv("SNH_ELEM_VARIANT")) c->elem_variant = saved;
     rep.elem_variant = c->elem_variant;
