@@ -37,6 +37,7 @@
 #include "../../include/snac_hip.h"
 #include "snh_kernels.h"
 #include "snh_landing.h"
+#include "snh_layout.h"
 
 using namespace snh;
 
@@ -689,8 +690,8 @@ __device__ __forceinline__ void store_density_at(const StepArgs& a, const DevMat
 }
 
 /* base[off / 8] for a uniform base and a per-lane byte offset below 4 GB (a
-   row of E or N doubles: device memory holds fewer than 2^29 elements): the
-   load takes its base from scalar registers and its offset from one vector
+   row of at most ROW_MOST doubles, which the choice of the kernel sees to: a
+   wrapped offset would read another node without a fault): the load takes its base from scalar registers and its offset from one vector
    register, so a row costs no vector address arithmetic */
 typedef const __attribute__((address_space(1))) char* gbase;   /* uniform, in global memory */
 __device__ __forceinline__ gbase row_base(const double* p) { return (gbase)(uintptr_t)p; }
@@ -845,7 +846,6 @@ __device__ __forceinline__ void tet_law(const StepArgs& a, const DevMaterial& m,
    carry no tet: they mirror tet 0 of element slot 0 but never write LDS or
    memory).  A lane's place in the ten tets' rows of a component must fit 32
    bits of byte offset: at most LANE_MOST_ELEMENTS elements. */
-#define LANE_MOST_ELEMENTS 53687091
 template <int RSET, bool MM>
 __device__ __forceinline__ void elem_pass(StepArgs a, const int blk, const int nblk) {
     __shared__ double sh_a[EPW][NTET];
@@ -4068,11 +4068,11 @@ static int launch_elem_args(snh_context* c, StepArgs a) {
 static int launch_elem_fp64(snh_context* c, StepArgs a) {
     dim3 grid((c->E + EPW - 1) / EPW), block(64);
     const bool mm = a.mat != nullptr;
+    const int32_t layout = elem_layout(c->elem_variant, c->N, c->E);
     /* the diagnostics are written by the element-per-lane variant only */
-    if (a.diag || c->elem_variant == SNH_ELEM_ELEMENT_PER_LANE ||
-        c->elem_variant == SNH_ELEM_ELEMENT_PER_LANE_LOWREG) {
+    if (a.diag || layout == SNH_ELEM_ELEMENT_PER_LANE || layout == SNH_ELEM_ELEMENT_PER_LANE_LOWREG) {
         dim3 g2((c->E + ELEM_BLOCK - 1) / ELEM_BLOCK), b2(ELEM_BLOCK);
-        const bool lr = !a.diag && c->elem_variant == SNH_ELEM_ELEMENT_PER_LANE_LOWREG;
+        const bool lr = !a.diag && layout == SNH_ELEM_ELEMENT_PER_LANE_LOWREG;
 #define SEQ_LAUNCH(R)                                                                         \
     do {                                                                                      \
         if (mm) {                                                                             \
@@ -4094,7 +4094,7 @@ static int launch_elem_fp64(snh_context* c, StepArgs a) {
         HIPCHK(hipGetLastError());
         return SNH_OK;
     }
-    const bool tw = c->elem_variant == SNH_ELEM_TET_PER_WAVE || c->E > LANE_MOST_ELEMENTS;
+    const bool tw = layout == SNH_ELEM_TET_PER_WAVE;
     if (tw) grid = dim3((c->E + 63) / 64);
     /* the waves are those of the instantiation launched: a mix of laws takes
        the kernel of all four, whatever is in the mix */
@@ -5185,7 +5185,8 @@ static void ens_free(snh_ensemble* e) {
    branches, each in its autotuned layout and overlapping on the hardware
    queues, are as fast or faster (64 models of 53k elements on average: FP64
    1.03x, mixed 1.10x the batched launches).  SNH_ENSEMBLE_BATCH=1 in the
-   environment batches whatever the sizes, =0 never. */
+   environment batches whatever the sizes that the batched passes can address
+   (batch_addressable), =0 never. */
 static bool ens_batchable(const std::vector<snh_context*>& m) {
     const char* env = getenv("SNH_ENSEMBLE_BATCH");
     if (env && env[0] == '0') return false;
@@ -5201,6 +5202,7 @@ static bool ens_batchable(const std::vector<snh_context*>& m) {
             (c->mat != nullptr) != (c0->mat != nullptr))
             return false;
         if (c->diag_on || c->beta_dens || c->thermal || c->node_variant != SNH_NODE_PER_NODE) return false;
+        if (!batch_addressable(c->N, c->E)) return false;
         if (c->cfg.precision == SNH_PRECISION_MIXED && c->mat) return false;
     }
     return true;
