@@ -1542,21 +1542,35 @@ __device__ __forceinline__ int gather_node(const StepArgs& a, int g, int& i, int
    32 after (j, k-1): with the 16384 nodes that an XCD's registers hold, a
    quarter and half a life for rows of 256 nodes, so that the four readings
    fall together and three of them hit L2.  Fetched from beyond L2 at
-   256x64x128 elements: 2.85 GB in bands of 8 without the turn, 1.65 GB so; the
-   pass 566 -> 545 us there, 465 -> 442 us at 192x48x192 and 122 -> 113 us at
-   130x35x97, where a turn of one row gives 543, 446 and 117 us.  A bijection
-   of the rows. */
+   256x64x128 elements: 2.85 GB in bands of 8 without the turn, 1.65 GB so.
+   Longer rows part the readings further than in bands of 8 without the turn,
+   and over few rows along y the turn wraps.  The pass, in bands of 8 / turned
+   (us): 268 / 271 at rows of 33 nodes, 262 / 262 at 65, 264 / 257 at 97,
+   258 / 252 at 129, 251 / 249 at 257, 252 / 256 at 289, 253 / 264 at 449,
+   247 / 275 at 513 and 241 / 310 at 1001 (65 rows along y, 1e6 nodes); at rows
+   of 257 nodes 250 / 254 with 13 rows along y, 253 / 251 with 21 and 262 / 253
+   with 33; 564 / 542 at 256x64x128.  So TURN_LEAST to TURN_MOST nodes in rows
+   of which y has TURN_LEAST_J or more are turned, others taken in bands; the
+   mixed gather's figures lie alike (586 / 561 at 256x64x128, 259 / 280 at rows
+   of 513).  The order with a turn of zero is that of the bands, from the same
+   instructions.  Bands of another height than the default (SNH_NODE_BAND) are
+   not turned.  A bijection of the rows. */
+#define NODE_BAND 8
 #define GATHER_BAND 16
+#define TURN_LEAST 88
+#define TURN_MOST 288
+#define TURN_LEAST_J 24
 __device__ __forceinline__ int gather_node_turned(const StepArgs& a, int g, int& i, int& j, int& k) {
     const int r = (int)fastdiv((uint32_t)g, a.dI);
     i = g - r * a.I;
-    const int b = (int)fastdiv((uint32_t)(r / GATHER_BAND), a.dJ);   /* r / (GATHER_BAND J) */
-    const int rem = r - b * GATHER_BAND * a.J;
-    const int planes = min(GATHER_BAND, a.K - b * GATHER_BAND);
-    j = planes == GATHER_BAND ? rem / GATHER_BAND : rem / planes;
+    const int KB = a.node_band;
+    const int b = (int)fastdiv((uint32_t)r, a.dPer);   /* r / (J KB) */
+    const int rem = r - b * KB * a.J;
+    const int planes = min(KB, a.K - b * KB);
+    j = planes == KB ? (int)fastdiv((uint32_t)rem, a.dKB) : rem / planes;
     const int q = rem - j * planes;
-    k = b * GATHER_BAND + q;
-    for (j -= 2 * q; j < 0;) j += a.J;
+    k = b * KB + q;
+    for (j -= a.node_turn * q; j < 0;) j += a.J;
     return i + a.I * (j + a.J * k);
 }
 
@@ -3126,7 +3140,7 @@ struct BatchMember {
     int64_t part_min;
     int64_t part_vmax;
     int64_t scal;
-    int32_t I, J, K, EI, EJ, EK, N, E, dtType, node_band, node_kc;
+    int32_t I, J, K, EI, EJ, EK, N, E, dtType, node_band, node_turn, node_kc;
     FastDiv dI, dJ, dEI, dEJ, dKB, dPer;   /* StepArgs' divisors */
     double gravity, demf, strain_inert, c_wave;
 };
@@ -3188,6 +3202,7 @@ __device__ __forceinline__ StepArgs member_args(const StepArgs& base, const Batc
     a.E = d.E;
     a.dtType = d.dtType;
     a.node_band = d.node_band;
+    a.node_turn = d.node_turn;
     a.node_kc = d.node_kc;
     a.gravity = d.gravity;
     a.demf = d.demf;
@@ -3516,6 +3531,16 @@ static void set_divisors(StepArgs& a) {
     a.dPer = fastdiv_make((uint32_t)(a.node_band > 0 ? a.J * a.node_band : 1));
 }
 
+/* the row order of the per-node gathers (gather_node_turned), which differs
+   from that of the other node kernels; a band of one plane is the plain
+   order */
+static void set_gather_order(StepArgs& a) {
+    const bool turn = a.node_band == NODE_BAND && a.I >= TURN_LEAST && a.I <= TURN_MOST && a.J >= TURN_LEAST_J;
+    a.node_turn = turn ? 2 : 0;
+    a.node_band = turn ? GATHER_BAND : std::max(a.node_band, 1);
+    set_divisors(a);
+}
+
 static StepArgs make_args(snh_context* c) {
     StepArgs a;
     a.xc = c->x[c->cur];
@@ -3556,6 +3581,7 @@ static StepArgs make_args(snh_context* c) {
     a.N = c->N; a.E = c->E;
     a.dtType = c->cfg.dtType;
     a.node_band = c->node_band;
+    a.node_turn = 0;
     a.node_kc = c->node_kc;
     a.gravity = c->cfg.gravity;
     a.demf = c->cfg.demf;
@@ -3815,7 +3841,7 @@ extern "C" int snh_context_create(const snh_config* cfg, snh_context** out) {
     }
     c->cur = 0;
     c->elem_variant = default_elem_variant(c->rset, c->E);
-    c->node_band = 8;
+    c->node_band = NODE_BAND;
     c->node_variant = SNH_NODE_PER_NODE;
     if (const char* nv = getenv("SNH_NODE_VARIANT")) c->node_variant = atoi(nv) == SNH_NODE_TILED ? SNH_NODE_TILED : SNH_NODE_PER_NODE;
     if (const char* nb = getenv("SNH_NODE_BAND")) c->node_band = atoi(nb);
@@ -4148,10 +4174,12 @@ static void launch_node_fp64(snh_context* c, const StepArgs& a) {
     }
     if (a.N > SLOT_MOST_NODES) {
         const dim3 g(c->n_node_blocks), b(NODE_BLOCK);
-        if (a.dens && a.mat) hipLaunchKernelGGL((k_node<true, true>), g, b, 0, c->stream, a);
-        else if (a.dens) hipLaunchKernelGGL((k_node<false, true>), g, b, 0, c->stream, a);
-        else if (a.mat) hipLaunchKernelGGL((k_node<true, false>), g, b, 0, c->stream, a);
-        else hipLaunchKernelGGL((k_node<false, false>), g, b, 0, c->stream, a);
+        StepArgs o = a;
+        set_gather_order(o);
+        if (a.dens && a.mat) hipLaunchKernelGGL((k_node<true, true>), g, b, 0, c->stream, o);
+        else if (a.dens) hipLaunchKernelGGL((k_node<false, true>), g, b, 0, c->stream, o);
+        else if (a.mat) hipLaunchKernelGGL((k_node<true, false>), g, b, 0, c->stream, o);
+        else hipLaunchKernelGGL((k_node<false, false>), g, b, 0, c->stream, o);
         c->n_vmax_parts = c->n_node_blocks;
         return;
     }
@@ -4176,7 +4204,9 @@ static int launch_node(snh_context* c, int refStep) {
     if (si >= 0 && c->sched_damp) a.damp_sched = c->sched_damp + (size_t)si * c->N;
     if (c->recording) a.tape_code = c->rec_code;
     if (c->cfg.precision == SNH_PRECISION_MIXED) {
-        hipLaunchKernelGGL(k_node_mx, dim3(c->n_node_blocks), dim3(NODE_BLOCK), 0, c->stream, a);
+        StepArgs m = a;
+        set_gather_order(m);
+        hipLaunchKernelGGL(k_node_mx, dim3(c->n_node_blocks), dim3(NODE_BLOCK), 0, c->stream, m);
         c->n_vmax_parts = c->n_node_blocks;
     } else {
         launch_node_fp64(c, a);
@@ -5291,6 +5321,7 @@ static int ens_batch_tables(snh_ensemble* e, EnsGroup& grp) {
             const int cur = c->cur;
             c->cur = e->cur0[grp.idx[i]] ^ q;
             args[i] = make_args(c);
+            if (c->cfg.precision == SNH_PRECISION_MIXED) set_gather_order(args[i]);
             c->cur = cur;
         }
         const StepArgs& b = args[0];
@@ -5344,6 +5375,7 @@ static int ens_batch_tables(snh_ensemble* e, EnsGroup& grp) {
             d.E = a.E;
             d.dtType = a.dtType;
             d.node_band = a.node_band;
+            d.node_turn = a.node_turn;
             d.node_kc = a.node_kc;
             d.gravity = a.gravity;
             d.demf = a.demf;
