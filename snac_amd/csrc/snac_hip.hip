@@ -4153,12 +4153,13 @@ static int sched_index(const snh_context* c, uint32_t t) {
     return (int)(t - c->sched_base);
 }
 
-/* Up to this many nodes the eight-wave gather is the faster one (it runs a
-   node's eight elements side by side: 10.5 us against 20.5 us at 16x8x16
-   elements, 41 / 45 us at 63x31x65, 69 / 77 us at 127x31x65); beyond, every CU
-   has waves enough and its block overhead shows (122 / 118 us at 462000 nodes,
-   616 / 566 us at 256x64x128). */
-#define SLOT_MOST_NODES 400000
+/* Up to this many nodes the eight-wave gather is the faster one: it runs a
+   node's eight elements side by side.  Beyond, every CU has waves enough and
+   its block overhead shows.  Per node / eight waves (us): 20.8 / 13.8 at 18500
+   nodes, 46 / 40 at 135000, 70 / 69 at 270000, 87 / 85 at 342000, 91 / 96 at
+   381000, 111 / 116 at 462000; with tet densities 80 / 78 at 270000,
+   101 / 99 at 342000, 106 / 112 at 381000, 133 / 148 at 461000. */
+#define SLOT_MOST_NODES 350000
 
 /* the FP64 node pass in the context's variant; records how many block
    maxima of |v| it leaves for k_fin */
