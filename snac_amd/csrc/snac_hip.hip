@@ -3607,19 +3607,6 @@ static void free_all(snh_context* c) {
         if (p) (void)hipFree(p);
 }
 
-/* The element-pass layout of a context that is not autotuned.  Tet per wave
-   fills its loads, tet per lane starts more and smaller blocks and lets fewer
-   tets wait for one that yields.  Measured (us, tet per lane / per wave):
-   elastic 9.5 / 10.7 at 8112 elements, 14.2 / 12.0 at 16384, 52 / 38 at
-   127000; Maxwell 11.1 / 12.9, 16.5 / 14.2, 65 / 50; Mohr-Coulomb extension
-   98 / 102 at 256000, 177 / 179 at 441000, 397 / 364 at 885000, and yielding
-   throughout 106 / 136, 199 / 236, 430 / 424; visco-plastic 111 / 117,
-   197 / 209, 473 / 429. */
-static int32_t default_elem_variant(int rset, int E) {
-    const bool soft = (rset & (RS_PLASTIC | RS_VISCOPLASTIC)) != 0;
-    return E >= (soft ? 700000 : 12000) ? SNH_ELEM_TET_PER_WAVE : SNH_ELEM_TET_PER_LANE;
-}
-
 extern "C" int snh_context_create(const snh_config* cfg, snh_context** out) {
     if (!cfg || !out) return set_err(SNH_EINVAL, "snh_context_create: null argument");
     *out = nullptr;
@@ -3840,7 +3827,7 @@ extern "C" int snh_context_create(const snh_config* cfg, snh_context** out) {
         return rc;
     }
     c->cur = 0;
-    c->elem_variant = default_elem_variant(c->rset, c->E);
+    c->elem_variant = default_elem_variant((c->rset & RS_PLASTIC) != 0, (c->rset & RS_VISCOPLASTIC) != 0, c->EI, c->E);
     c->node_band = NODE_BAND;
     c->node_variant = SNH_NODE_PER_NODE;
     if (const char* nv = getenv("SNH_NODE_VARIANT")) c->node_variant = atoi(nv) == SNH_NODE_TILED ? SNH_NODE_TILED : SNH_NODE_PER_NODE;

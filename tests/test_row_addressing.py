@@ -21,11 +21,14 @@ def rules(tmp_path_factory):
     d = tmp_path_factory.mktemp("layout")
     (d / "l.c").write_text('#include "snh_layout.h"\n'
                            "int layout(int v, long long N, long long E) { return elem_layout(v, N, E); }\n"
+                           "int untuned(int p, int v, long long EI, long long E)"
+                           " { return default_elem_variant(p, v, EI, E); }\n"
                            "int batch(long long N, long long E) { return batch_addressable(N, E); }\n")
     subprocess.check_call(["gcc", "-shared", "-fPIC", "-I", os.path.join(ROOT, "snac_amd", "csrc"), "-o",
                            str(d / "l.so"), str(d / "l.c")])
     lib = C.CDLL(str(d / "l.so"))
     lib.layout.argtypes = [C.c_int, C.c_longlong, C.c_longlong]
+    lib.untuned.argtypes = [C.c_int, C.c_int, C.c_longlong, C.c_longlong]
     lib.batch.argtypes = [C.c_longlong, C.c_longlong]
     return lib
 
@@ -49,3 +52,16 @@ def test_offsets_fit_32_bits(rules, nodes):
             assert got == v   # a layout that can address the mesh stays
     if rules.batch(N, E):
         assert _largest_offset(LANE, N, E) < 1 << 32 and _largest_offset(WAVE, N, E) < 1 << 32
+
+
+# (plastic, visco-plastic, elements along x, elements): the faster layout of
+# an untuned context, as measured
+UNTUNED = [((0, 0, 16, 8112), LANE), ((0, 0, 32, 16384), WAVE), ((0, 0, 8, 819200), WAVE),
+           ((1, 0, 100, 441000), LANE), ((1, 0, 192, 884736), WAVE), ((1, 0, 64, 800000), WAVE),
+           ((1, 0, 8, 819200), LANE), ((1, 0, 16, 819200), LANE), ((1, 0, 48, 825600), LANE),
+           ((1, 0, 16, 2048000), WAVE), ((0, 1, 8, 819200), WAVE), ((0, 1, 100, 441000), LANE)]
+
+
+@pytest.mark.parametrize("case,layout", UNTUNED, ids=str)
+def test_untuned_layout(rules, case, layout):
+    assert rules.untuned(*case) == layout
