@@ -7,9 +7,9 @@
  * page fault of the caller's new array.  Here the DMA engine fills pinned
  * chunks at the link's rate while several threads carry the chunks that have
  * landed into the caller's array, faults included.  The chunks belong to the
- * process (at most LAND_CHUNKS of them, allocated by the first large download
- * and given back with the last context); a download that finds too few of
- * them free, or no threads, takes the plain copy.
+ * process (at most LAND_CHUNKS of them, allocated when downloads are large or
+ * have repeated, LAND_ALLOC, and given back with the last context); a download
+ * that finds too few of them free, or no threads, takes the plain copy.
  */
 #ifndef SNH_LANDING_H
 #define SNH_LANDING_H
@@ -27,12 +27,20 @@
 #define LAND_THREADS 8
 /* below this a plain copy is as fast (the threads cost 0.1 ms to start) */
 #define LAND_LEAST ((size_t)8 << 20)
+/* Allocating the chunks costs 1.5-2 ms, and as much again is lost to the copies
+   after they are given back, which a download of less than LAND_ALLOC does not
+   earn: the first of a context that is the process's only one took 2.4 ms for
+   13 MB and 2.9 ms for 31 MB, against 1.1 and 2.5 with the plain copy (63 MB:
+   4.2 against 6.9).  So chunks are allocated for a larger download, or when the
+   smaller ones together have come to twice that. */
+#define LAND_ALLOC ((size_t)40 << 20)
 
 struct LandPool {
     std::mutex mu;
     void* chunk[LAND_CHUNKS] = {};
     bool used[LAND_CHUNKS] = {};
     int contexts = 0;
+    size_t plain = 0;   /* bytes copied plainly for want of chunks */
 };
 static LandPool g_land;
 
@@ -44,6 +52,7 @@ static void land_context_made() {
 static void land_context_gone() {
     std::lock_guard<std::mutex> l(g_land.mu);
     if (--g_land.contexts > 0) return;
+    g_land.plain = 0;
     for (int k = 0; k < LAND_CHUNKS; k++)
         if (g_land.chunk[k] && !g_land.used[k]) {
             (void)hipHostFree(g_land.chunk[k]);
@@ -117,6 +126,9 @@ class Landing {
     void open(size_t total) {
         {
             std::lock_guard<std::mutex> l(g_land.mu);
+            int have = 0;
+            for (int k = 0; k < LAND_CHUNKS; k++) have += g_land.chunk[k] && !g_land.used[k];
+            if (have < LAND_SLOTS && total < LAND_ALLOC && (g_land.plain += total) < 2 * LAND_ALLOC) return;
             int n = 0;
             for (int k = 0; k < LAND_CHUNKS && n < LAND_SLOTS; k++) {
                 if (g_land.used[k]) continue;
@@ -146,7 +158,6 @@ class Landing {
             ok = !th_.empty();
         }
         open_ = ok;
-        (void)total;
     }
     void carry(int t) {
         size_t T;
