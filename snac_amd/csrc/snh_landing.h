@@ -20,6 +20,7 @@
 #include <condition_variable>
 #include <mutex>
 #include <thread>
+#include <vector>
 
 #define LAND_CHUNK ((size_t)4 << 20)
 #define LAND_SLOTS 4      /* chunks of one download */
@@ -145,7 +146,11 @@ class Landing {
         }
         bool ok = slots_ == LAND_SLOTS;
         for (int s = 0; s < LAND_SLOTS && ok; s++)
-            ok = hipEventCreateWithFlags(&job_[s].landed, hipEventDisableTiming) == hipSuccess;
+            if (hipEventCreateWithFlags(&job_[s].landed, hipEventDisableTiming) != hipSuccess) {
+                job_[s].landed = nullptr;
+                (void)hipGetLastError();   /* not the next launch's error */
+                ok = false;
+            }
         if (ok) {
             const int T = land_threads();
             try {
