@@ -69,7 +69,9 @@ static int land_threads() {
     return n;
 }
 
-/* One download: push() the fields in stream order, finish() once. */
+/* One download: push() the fields in stream order, finish() once.  The chunks
+   are pinned for every device, since contexts of several may take turns at
+   them. */
 class Landing {
   public:
     Landing(hipStream_t stream, size_t total) : stream_(stream) {
@@ -133,7 +135,7 @@ class Landing {
             int n = 0;
             for (int k = 0; k < LAND_CHUNKS && n < LAND_SLOTS; k++) {
                 if (g_land.used[k]) continue;
-                if (!g_land.chunk[k] && hipHostMalloc(&g_land.chunk[k], LAND_CHUNK, hipHostMallocDefault) != hipSuccess) {
+                if (!g_land.chunk[k] && hipHostMalloc(&g_land.chunk[k], LAND_CHUNK, hipHostMallocPortable) != hipSuccess) {
                     g_land.chunk[k] = nullptr;
                     (void)hipGetLastError();
                     break;

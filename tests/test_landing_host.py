@@ -1,7 +1,7 @@
 """The download path of snac_amd/csrc/snh_landing.h compiled for the host, its
 HIP calls replaced by ones that copy at once, count and fail when told to:
 every byte lands, for all sizes around a chunk and around the part of a
-thread; a download for which events or
+thread; the chunks are pinned for every device; a download for which events or
 pinned memory are refused takes the plain copy and leaves no error behind for
 the next launch to find; chunks are allocated, bounded and given back as the
 header says; a download without a copy waits for the stream."""
@@ -22,12 +22,13 @@ typedef void* hipStream_t;
 typedef int* hipEvent_t;
 enum { hipSuccess = 0, hipErrorOutOfMemory = 2, hipMemcpyDeviceToHost = 2, hipEventDisableTiming = 2,
        hipHostMallocDefault = 0, hipHostMallocPortable = 1 };
-static std::atomic<int> mallocs{0}, frees{0}, events{0}, copies{0}, waits{0};
+static std::atomic<int> mallocs{0}, frees{0}, not_portable{0}, events{0}, copies{0}, waits{0};
 static int fail_malloc_at = -1, fail_event_at = -1;
 static thread_local hipError_t last = hipSuccess;
 static hipError_t hipGetLastError() { hipError_t e = last; last = hipSuccess; return e; }
-static hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+static hipError_t hipHostMalloc(void** p, size_t n, unsigned flags) {
     if (mallocs++ == fail_malloc_at) return last = hipErrorOutOfMemory;
+    if (!(flags & hipHostMallocPortable)) not_portable++;
     return (*p = malloc(n)) ? hipSuccess : hipErrorOutOfMemory;
 }
 static hipError_t hipHostFree(void* p) { frees++; free(p); return hipSuccess; }
@@ -83,6 +84,7 @@ int main() {
             WANT(land(n, s, 48 * MB));
     WANT(mallocs - frees <= LAND_CHUNKS + 1);   /* one was refused */
     land_context_gone();
+    WANT(not_portable == 0);
     /* chunks only when downloads are worth them */
     land_context_made();
     const int m0 = mallocs;
