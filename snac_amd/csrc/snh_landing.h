@@ -69,6 +69,16 @@ static int land_threads() {
     return n;
 }
 
+/* bytes a to b of the n that go to dst are thread t's of T.  Parts end at page
+   boundaries of the destination, so that no two threads fault one page. */
+static void land_part(const char* dst, size_t n, size_t T, size_t t, size_t* a, size_t* b) {
+    const size_t page = 4096, into = (uintptr_t)dst % page;
+    const size_t part = ((n + into + T - 1) / T + page - 1) / page * page;   /* in pages from dst's own */
+    const size_t lo = part * t, hi = part * (t + 1);
+    *a = t == 0 || lo <= into ? 0 : (lo - into < n ? lo - into : n);
+    *b = t + 1 == T || hi - into > n ? n : hi - into;
+}
+
 /* One download: push() the fields in stream order, finish() once.  The chunks
    are pinned for every device, since contexts of several may take turns at
    them. */
@@ -181,10 +191,8 @@ class Landing {
             }
             const hipError_t r = hipEventSynchronize(j.landed);
             if (r != hipSuccess) error_ = (int)r;
-            /* page-sized parts, so that no two threads fault one page */
-            const size_t part = (j.bytes / T + 4095) & ~(size_t)4095;
-            const size_t a = part * t < j.bytes ? part * t : j.bytes;
-            const size_t b = t + 1 == (int)T || part * (t + 1) > j.bytes ? j.bytes : part * (t + 1);
+            size_t a, b;
+            land_part(j.dst, j.bytes, T, (size_t)t, &a, &b);
             if (r == hipSuccess && b > a) memcpy(j.dst + a, (char*)slot_[i % LAND_SLOTS] + a, b - a);
             bool last;
             {

@@ -103,6 +103,20 @@ int main() {
         const int w = waits;
         WANT(l.finish() == hipSuccess && waits == w + 1);
     }
+    /* the threads' parts cover a chunk once and part it at page boundaries */
+    for (size_t n : {(size_t)4, (size_t)8, (size_t)4095, (size_t)4096, (size_t)70000, C - 8, C})
+        for (uintptr_t d : {(uintptr_t)0x7f0000000000, (uintptr_t)0x7f0000000010, (uintptr_t)0x7f0000000ff8})
+            for (size_t T : {1, 3, 8}) {
+                size_t at = 0;
+                for (size_t t = 0; t < T; t++) {
+                    size_t a, b;
+                    land_part((char*)d, n, T, t, &a, &b);
+                    WANT(a == at && b >= a && b <= n);
+                    WANT(b == n || (d + b) % 4096 == 0);
+                    at = b;
+                }
+                WANT(at == n);
+            }
     printf("bad %d\n", bad);
     return bad != 0;
 }
