@@ -240,13 +240,14 @@ SNH_HD void tet_kinematics(const double X[4][3], const double U[4][3], TetKin& o
     const double s12 = T_(0, 1, 2) + T_(1, 1, 2) + T_(2, 1, 2) + T_(3, 1, 2);
     /* x / 3.0 / V as two correctly rounded quotients */
     const snh_recip rV = snh_recip_make(V);
+    const double hv = -(snh_recip_rn(rV) * 0.25);   /* RN(0.5/V) == RN(1/V)/2; a quarter for the doubled products */
+    /* (before the quotients: after them it costs the Mohr-Coulomb pass 0.5 %) */
     o.sr[0] = snh_quot(snh_ndiv6(s00), rV);
     o.sr[1] = snh_quot(snh_ndiv6(s11), rV);
     o.sr[2] = snh_quot(snh_ndiv6(s22), rV);
     o.sr[3] = snh_quot(snh_ndiv12(s01 + T_(0, 1, 0) + T_(1, 1, 0) + T_(2, 1, 0) + T_(3, 1, 0)), rV);
     o.sr[4] = snh_quot(snh_ndiv12(s02 + T_(0, 2, 0) + T_(1, 2, 0) + T_(2, 2, 0) + T_(3, 2, 0)), rV);
     o.sr[5] = snh_quot(snh_ndiv12(s12 + T_(0, 2, 1) + T_(1, 2, 1) + T_(2, 2, 1) + T_(3, 2, 1)), rV);
-    const double hv = -(rV.hi * 0.25);   /* RN(0.5/V) == RN(1/V)/2; a quarter for the doubled products */
     o.w[0] = snh_div3(hv * (s01 - T_(0, 1, 0) - T_(1, 1, 0) - T_(2, 1, 0) - T_(3, 1, 0)));
     o.w[1] = snh_div3(hv * (s02 - T_(0, 2, 0) - T_(1, 2, 0) - T_(2, 2, 0) - T_(3, 2, 0)));
     o.w[2] = snh_div3(hv * (s12 - T_(0, 2, 1) - T_(1, 2, 1) - T_(2, 2, 1) - T_(3, 2, 1)));

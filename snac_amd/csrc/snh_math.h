@@ -35,12 +35,15 @@ SNH_HD int snh_iadd_wrap(int a, int b) { return (int)((unsigned)a + (unsigned)b)
  * floating-point division when the divisor is known in advance", IEEE Trans.
  * Computers 53 (2004), method 1).  The sum before the rounding is within
  * 2^-52 ulp of a / b, so the result is RN(a / b) unless the quotient lies that
- * close to a rounding midpoint; 4e9 random quotients on gfx950 gave no
- * difference from the division.  Normal range only.
+ * close to a rounding midpoint.  That takes a dividend and a divisor made for
+ * it: 2^n over the largest number below a power of two, and one pair besides
+ * in 1.7e7 built near such midpoints; 4e9 random quotients on gfx950 gave no
+ * difference from the division.  Either sign of b; normal range only.
  *
- * From an estimate of 1 / b good to 2^-24 (v_rcp_f64, v_rsq_f64), one or two
+ * From an estimate of 1 / b good to 2^-23 (v_rcp_f64, v_rsq_f64), one or two
  * Newton steps (P. Markstein, 1990) make hi faithful; the residual
- * 1 - b hi is then exact, and lo is its product with hi. */
+ * 1 - b hi is then exact, and lo is its product with hi.  hi itself is RN(1/b)
+ * for all but a few b just below a power of two: snh_recip_rn gives that. */
 typedef struct {
     double hi, lo;
 } snh_recip;
@@ -54,29 +57,34 @@ SNH_HD snh_recip snh_recip_of(double b, double y) {
 }
 SNH_HD double snh_quot(double a, snh_recip r) { return fma(a, r.hi, a * r.lo); }
 
-/* the reciprocal of b > 0 */
+/* RN(1 / b).  For b = 2 - k 2^-52 (times a power of two) with a small odd k,
+ * 1 / b lies k^2 2^-54 ulp beyond a midpoint, so hi, the nearest to within
+ * 2^-49 ulp, may be the number on the other side, and for k = 1 so may the
+ * rounded sum hi + lo; a 2^-105 part of hi more settles that case and is too
+ * little to matter in any other. */
+SNH_HD double snh_recip_rn(snh_recip r) { return r.hi + fma(r.hi, 0x1p-105, r.lo); }
+
+/* the pair from an estimate y of 1 / b good to 2^-23 */
+SNH_HD snh_recip snh_recip_refine(double b, double y) { return snh_recip_of(b, fma(fma(-b, y, 1.0), y, y)); }
 SNH_HD snh_recip snh_recip_make(double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    double y = __builtin_amdgcn_rcp(b);
-    y = fma(fma(-b, y, 1.0), y, y);
+    return snh_recip_refine(b, __builtin_amdgcn_rcp(b));
 #else
-    const double y = 1.0 / b;
+    return snh_recip_refine(b, 1.0 / b);
 #endif
-    return snh_recip_of(b, y);
 }
 
-/* RN(sqrt(x)) for x > 0 and, in r, the reciprocal of that root.  Goldschmidt's
- * coupled iteration for sqrt(x) and 1 / (2 sqrt(x)) from v_rsq_f64, then two
- * residual corrections of the root (Markstein 1990; Muller et al., Handbook of
- * Floating-Point Arithmetic, 2nd ed., sec. 4.7), which give the correctly
- * rounded root; the reciprocal comes out of the same iteration instead of a
- * division.  Without the scaling of the library's sqrt: normal range only
- * (x = 0 gives NaN, as the 0 / 0 of a face without area does).
- * 13 instructions for root and reciprocal and 2 per quotient, against 31 and
- * 5 with sqrt, 1 / s and snh_div_by. */
-SNH_HD double snh_sqrt_recip(double x, snh_recip* r) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const double y = __builtin_amdgcn_rsq(x);
+/* RN(sqrt(x)) for x > 0 and, in r, the reciprocal of that root, from an
+ * estimate y of 1 / sqrt(x) good to 2^-23.  Goldschmidt's coupled iteration
+ * for sqrt(x) and 1 / (2 sqrt(x)), then two residual corrections of the root
+ * (Markstein 1990; Muller et al., Handbook of Floating-Point Arithmetic, 2nd
+ * ed., sec. 4.7), which give the correctly rounded root; the reciprocal comes
+ * out of the same iteration instead of a division.  Without the scaling of the
+ * library's sqrt: x from 2^-900 to 2^1000 (x = 0 gives NaN, as the 0 / 0 of a
+ * face without area does).  13 instructions for root and reciprocal and 2 per
+ * quotient, against 31 and 5 with sqrt, 1 / s and quotients corrected twice by
+ * their residual. */
+SNH_HD double snh_sqrt_refine(double x, double y, snh_recip* r) {
     double g = x * y, h = 0.5 * y;
     const double t = fma(-h, g, 0.5);
     g = fma(g, t, g);
@@ -87,10 +95,12 @@ SNH_HD double snh_sqrt_recip(double x, snh_recip* r) {
     g = fma(d, h, g);
     *r = snh_recip_of(g, h + h);
     return g;
+}
+SNH_HD double snh_sqrt_recip(double x, snh_recip* r) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return snh_sqrt_refine(x, __builtin_amdgcn_rsq(x), r);
 #else
-    const double s = sqrt(x);
-    *r = snh_recip_of(s, 1.0 / s);
-    return s;
+    return snh_sqrt_refine(x, 1.0 / sqrt(x), r);
 #endif
 }
 
