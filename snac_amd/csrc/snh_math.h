@@ -184,18 +184,4 @@ SNH_DIV3C(snh_div12, 0.25)
 SNH_DIV3C(snh_ndiv6, -0.5)
 SNH_DIV3C(snh_ndiv12, -0.25)
 
-/* RN(a / b) from y = RN(1 / b) (P. Markstein, "Computation of elementary
- * functions on the IBM RISC System/6000", IBM J. Res. Dev. 34 (1990); and
- * Muller et al., Handbook of Floating-Point Arithmetic, 2nd ed., sec. 4.7):
- * q0 = RN(a y) is within 1.5 ulp; one residual step makes it faithful; with
- * a faithful q and the correctly rounded reciprocal, r = a - b q is exact and
- * RN(q + r y) is the correctly rounded quotient.  Normal range only. */
-SNH_HD double snh_div_by(double a, double b, double y) {
-    double q = a * y;
-    double r = fma(-b, q, a);
-    q = fma(r, y, q);
-    r = fma(-b, q, a);
-    return fma(r, y, q);
-}
-
 #endif
