@@ -361,11 +361,18 @@ def _pmc_run(counters, args):
         shutil.rmtree(d, ignore_errors=True)
 
 
+# the kernels of a pass: which of them runs is a matter of size and precision
+# (the LDS-tiled node pass is left out: the autotuner alone launches it more
+# often than the few steps of a counter run launch the pass they use)
+_PASS_KERNELS = {"k_elem": ("k_elem", "k_elem_mx"), "k_node": ("k_node", "k_node_slot", "k_node_mx"),
+                 "k_geo": ("k_geo", "k_geo_tets")}
+
+
 def _kernel_rows(res, prefix):
-    """dispatches of the most-dispatched kernel whose name starts with prefix
-    (the variant the timed steps ran; the autotuner launches the others a
-    few times each)"""
-    names = [n for n in res if n.split("(")[0].split("<")[0].strip().endswith(prefix)]
+    """dispatches of the most-dispatched kernel of a pass (the variant the
+    timed steps ran; the autotuner launches the others a few times each)"""
+    kernels = _PASS_KERNELS.get(prefix, (prefix,))
+    names = [n for n in res if n.split("(")[0].split("<")[0].split()[-1].split("::")[-1] in kernels]
     if not names:
         return None, None
     name = max(names, key=lambda n: len(res[n]))
@@ -548,10 +555,12 @@ def main():
     if traffic:
         out["counters"] = traffic
         # HBM bytes the counters saw per element-step over the step's kernels
-        # (k_fin, one block, is left out), beside the compulsory bytes
-        measured = sum(traffic[k]["bytes"] for k in ("k_elem", "k_node", "k_geo") if k in traffic)
-        out["step_roofline"]["measured_bytes_per_element_step"] = measured / E
-        out["step_roofline"]["measured_over_compulsory"] = measured / E / step_bytes
+        # (k_fin, one block, is left out), beside the compulsory bytes; none
+        # if a pass was not seen
+        seen = all(k in traffic for k in _PASS_KERNELS)
+        measured = sum(traffic[k]["bytes"] for k in _PASS_KERNELS) / E if seen else None
+        out["step_roofline"]["measured_bytes_per_element_step"] = measured
+        out["step_roofline"]["measured_over_compulsory"] = measured / step_bytes if seen else None
 
     if not args.no_adjoint and args.precision == "fp64":
         from snac_amd import problem as P
