@@ -309,15 +309,16 @@ int snh_profile(snh_context* ctx, int enable);
 /* Kernel-variant autotuner (no counterpart in the reference).  Times each
  * candidate implementation of the element pass (one tet per lane, 6
  * elements per wave; one element per thread keeping the tet kinematics in
- * registers; the same recomputing them; one wave per tet index over 64
- * elements) on a scratch copy of the current state, a few launches
- * each, and keeps the fastest for this context.  Call after
+ * registers; the same recomputing them; 64 elements per block, whose waves
+ * take one or two of the ten tets of all of them) on a scratch copy of the
+ * current state, a few launches each, and keeps the fastest for this context.
+ * The times are those of a context that has the GPU to itself.  Call after
  * snh_timestep_zero; the state is not modified.  The choice can be forced
  * with the environment variable SNH_ELEM_VARIANT=0|1|2|3. */
 #define SNH_ELEM_TET_PER_LANE            0
 #define SNH_ELEM_ELEMENT_PER_LANE        1
 #define SNH_ELEM_ELEMENT_PER_LANE_LOWREG 2   /* kinematics recomputed, not kept */
-#define SNH_ELEM_TET_PER_WAVE            3   /* 64 elements per block, one wave per tet */
+#define SNH_ELEM_TET_PER_WAVE            3   /* 64 elements per block, one or two tets per wave */
 #define SNH_ELEM_VARIANTS                4
 #define SNH_NODE_TUNES 4   /* node pass: per node; tiled with 4, 8, 16 planes */
 typedef struct snh_tune_report {

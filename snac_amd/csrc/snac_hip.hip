@@ -965,18 +965,20 @@ __device__ __forceinline__ void elem_pass(StepArgs a, const int blk, const int n
    over 64 consecutive elements of one row and everything that depends on the
    tet is scalar.  Which, by the law, at 256x64x128 elements:
    - elastic, Maxwell: five waves, tets w and w + 5 one after the other; what
-     the second phase needs of the first tet waits in LDS.  At 96 registers and
-     41 KB three blocks share a CU and cover each other's loads and barriers:
+     the second phase needs of the first tet waits in LDS.  At 96 registers (2
+     or 3 of which spill) and 41 KB three blocks share a CU and cover each
+     other's loads and barriers:
      660 and 833 us, against 729 and 900 us with ten waves (one block a CU) and
      870 and 1020 us with ten waves and vector addresses;
    - the plastic laws: ten waves of one tet, up to 168 registers: 884 us
      Mohr-Coulomb and 1026 us visco-plastic, against 920 and 1075 us with five
      (their return diverges, and a wave then does it for both its tets) and
      1160 and 1445 us with ten waves held to 96 registers.
-   (The four take 658, 797, 860 and 1008 us with the later arithmetic.)
-   What bounds it now is the wait for its loads and barriers: at 884 us the
-   Mohr-Coulomb pass issues VALU instructions 35 % of the time and moves 2.4 GB
-   at 2.7 TB/s. */
+   (Elastic, Maxwell, Mohr-Coulomb and visco-plastic take 668, 836, 880 and 1035
+   us with the later arithmetic.)
+   What bounds it now is the wait for its loads and barriers: at 880 us the
+   Mohr-Coulomb pass issues VALU instructions 36 % of the time and moves 2.4 GB
+   at 2.7 TB/s, the elastic one 40 % and 2.3 GB at 3.4 TB/s. */
 __host__ __device__ constexpr int tw_waves(int rset) {
     return (rset & (RS_PLASTIC | RS_VISCOPLASTIC)) ? 10 : 5;
 }
