@@ -80,7 +80,7 @@ SNH_HD snh_recip snh_recip_make(double b) {
  * (Markstein 1990; Muller et al., Handbook of Floating-Point Arithmetic, 2nd
  * ed., sec. 4.7), which give the correctly rounded root; the reciprocal comes
  * out of the same iteration instead of a division.  Without the scaling of the
- * library's sqrt: x from 2^-900 to 2^1000 (x = 0 gives NaN, as the 0 / 0 of a
+ * library's sqrt: x from 2^-918 to 2^1023 (x = 0 gives NaN, as the 0 / 0 of a
  * face without area does).  13 instructions for root and reciprocal and 2 per
  * quotient, against 31 and 5 with sqrt, 1 / s and quotients corrected twice by
  * their residual. */

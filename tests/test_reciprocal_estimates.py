@@ -64,7 +64,7 @@ int main(void) {
         const double b = 2.0 - k * 0x1p-52;
         recip += snh_recip_rn(snh_recip_refine(b, estimate(1.0 / b))) != 1.0 / b;
     }
-    const double ends[] = {0x1p-900, 0x1.fffffffffffffp-900, 0x1.5p-899, 0x1p1000, 0x1.fffffffffffffp999, 0x1.7p999};
+    const double ends[] = {0x1p-918, 0x1.fffffffffffffp-918, 0x1.5p-917, 0x1p1022, 0x1.fffffffffffffp1021, 0x1.7p1022};
     for (int k = 0; k < 6; k++) {
         snh_recip rs;
         root += snh_sqrt_refine(ends[k], estimate(1.0 / sqrt(ends[k])), &rs) != sqrt(ends[k]);
